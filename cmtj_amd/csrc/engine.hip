@@ -117,15 +117,15 @@ static const KEntry* pick_kernel(int prec, int nl, int solver, uint32_t flags, u
   // automatic choice: on a batch too small to fill the chip, the time of a
   // sweep is its longest instance's step count times the latency of one
   // wave step.  One lane per component issues about half the instructions
-  // per wave step of one lane per layer, at four times the lanes: it wins
-  // while its waves still fit one per SIMD, and costs about twice the
-  // instructions per junction-step beyond that.
+  // per wave step of one lane per layer (111 against 199 VALU on the PIMM
+  // set), at four times the lanes: it wins while its waves still fit one per
+  // SIMD, and costs about twice the instructions per junction-step beyond that.
   if (lanes == CMTJ_LANES_AUTO && best[2] && n_inst * (uint64_t)best[2]->lpi <= 64 * kSimds) return best[2];
-  // one lane per layer for multilayer instances: on full-chip batches it
-  // measured no slower than one lane per instance (1M-instance CIMS ensemble
-  // 6.6e10 vs 6.3e10 junction-steps/s, 65,536-point PIMM sweep 2.56e10 vs
-  // 2.44e10 on MI355X): its register footprint is smaller, so more waves fit
-  // per SIMD.
+  // one lane per layer for multilayer instances: its register footprint is
+  // smaller than one lane per instance's, so more waves fit per SIMD, and the
+  // exact sets of large batches have their leanest kernels there (65,536-point
+  // PIMM sweep 6.5e10 junction-steps/s against 2.4e10 with one lane per
+  // instance, 131,072-instance CIMS ensemble 9.6e10 against 6.3e10).
   if (best[1] && (nl >= 2 || !best[0])) return best[1];
   if (best[0]) return best[0];
   return best[1] ? best[1] : best[2];

@@ -229,14 +229,25 @@ CMTJ_HD double driver_value(const cmtj_driver& d, double t) {
 
 // ---- Philox4x32-10 counter-based generator ---------------------------------
 
+// a ^ b ^ c in one instruction (truth table 0x96; the compiler leaves two xors)
+CMTJ_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#ifdef __HIP_DEVICE_COMPILE__
+  uint32_t r;
+  asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x96" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 CMTJ_HD void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
                            uint32_t k1, uint32_t out[4]) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
     const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-    const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+    const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+    const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
     c1 = (uint32_t)p1;
     c3 = (uint32_t)p0;
     c0 = n0;
@@ -248,6 +259,25 @@ CMTJ_HD void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, u
   out[1] = c1;
   out[2] = c2;
   out[3] = c3;
+}
+
+// sin and cos of 2 pi u for u in (0, 1]: the nearest quarter turn n/4 off
+// (exactly), minimax polynomials of the rest r in [-1/8, 1/8], quadrant by the
+// bits of n.  No range or class handling, which sincospif carries for other
+// arguments.
+__device__ __forceinline__ void sincos_turn(float u, float& s, float& c) {
+  const float t = fmaf(u, 4.0f, 12582912.0f);  // n in the low bits of 1.5 * 2^23 + n
+  const uint32_t n = __float_as_uint(t);
+  const float r = fmaf(t - 12582912.0f, -0.25f, u), z = r * r;
+  // (2 pi split in two so that its rounding does not enter; largest errors of
+  // the polynomials 3.2e-9 and 6.4e-11)
+  const float q = fmaf(z, fmaf(z, fmaf(z, -75.393562653f, 81.592353551f), -41.341661455f), -1.9519167e-07f);
+  const float sr = fmaf(r, 6.2831854820f, r * q);
+  const float cr = fmaf(z, fmaf(z, fmaf(z, fmaf(z, 59.229243562f, -85.443236277f), 64.939321847f), -19.739208682f), 1.0f);
+  const bool odd = (n & 1u) != 0u;
+  const float a = odd ? cr : sr, b = odd ? sr : cr;
+  s = __uint_as_float(__float_as_uint(a) ^ ((n << 30) & 0x80000000u));
+  c = __uint_as_float(__float_as_uint(b) ^ (((n + 1u) << 30) & 0x80000000u));
 }
 
 // Three N(0,1) draws of (step, layer) in the junction's stream: Box-Muller
@@ -276,16 +306,25 @@ __device__ __forceinline__ V3<float> thermal_normals<float>(uint64_t seed, uint6
   uint32_t o[4];
   philox4x32_10(step, layer, (uint32_t)stream, (uint32_t)(stream >> 32), (uint32_t)seed,
                 (uint32_t)(seed >> 32), o);
-  const float s = 2.3283064365386963e-10f;
-  const float u0 = ((float)o[0] + 0.5f) * s, u1 = ((float)o[1] + 0.5f) * s;
-  const float u2 = ((float)o[2] + 0.5f) * s, u3 = ((float)o[3] + 0.5f) * s;
-  // (float)o + 0.5 rounds to 2^32 for the top values; clamp below 1
-  const float one_m = 0.99999994f;
-  const float r0 = sqrtf(-2.0f * logf(fminf(u0, one_m)));
-  const float r1 = sqrtf(-2.0f * logf(fminf(u2, one_m)));
+  // (o + 0.5) 2^-32, the scaling exact, so one rounding; (float)o rounds to
+  // 2^32 for the top values: clamp below 1
+  const float s = 2.3283064365386963e-10f, one_m = 0.99999994f;
+  const float u0 = fminf(fmaf((float)o[0], s, 0.5f * s), one_m), u1 = fmaf((float)o[1], s, 0.5f * s);
+  const float u2 = fminf(fmaf((float)o[2], s, 0.5f * s), one_m), u3 = fmaf((float)o[3], s, 0.5f * s);
+  // sqrt(-2 ln u) for u in [2^-33, 1): no denormal, zero or infinity comes up,
+  // so the hardware's base-2 logarithm and reciprocal root with one correction
+  // take the place of logf and sqrtf with their range handling (26 -> 12
+  // instructions a value; over 3.3e8 u spread on the range: largest relative
+  // error 1.31e-7 against 1.50e-7, rms 3.54e-8 against 3.77e-8)
+  auto radius = [](float u) __attribute__((always_inline)) -> float {
+    const float x = -1.3862943611198906f * __builtin_amdgcn_logf(u);
+    const float y = __builtin_amdgcn_rsqf(x), r = x * y;
+    return fmaf(0.5f * fmaf(-r, r, x), y, r);
+  };
+  const float r0 = radius(u0), r1 = radius(u2);
   float s1, c1, s3, c3;
-  sincospif(2.0f * u1, &s1, &c1);
-  sincospif(2.0f * u3, &s3, &c3);
+  sincos_turn(u1, s1, c1);
+  sincos_turn(u3, s3, c3);
   return mk<float>(r0 * c1, r0 * s1, r1 * c3);
 }
 

@@ -1,7 +1,7 @@
 // registry.h -- kernel registry shared by the instantiation units.
 #pragma once
 
-#include "kernels_cl.h"
+#include "kernels_lx.h"
 
 namespace cmtj {
 
@@ -71,10 +71,10 @@ KTable kernels_group4();  // the same on four waves per group
   {PREC, L, L, S, FM, false, (const void*)&cmtj::k_junction_ll<R, L, S, FM, false>, \
    "k_junction_ll<" #R "," #L "," #S "," #FM ">"}
 
-// the same with the register allocation capped for WPE waves per SIMD
-#define CMTJ_KL_WPE(R, PREC, L, S, FM, WPE)                                              \
-  {PREC, L, L, S, FM, false, (const void*)&cmtj::k_junction_ll<R, L, S, FM, false, WPE>, \
-   "k_junction_ll<" #R "," #L "," #S "," #FM ",waves " #WPE ">"}
+// the large batches' exact sets (kernels_lx.h), the register allocation capped for WPE waves per SIMD
+#define CMTJ_KLX(R, PREC, L, S, FM, WPE, ND)                                                \
+  {PREC, L, L, S, FM, false, (const void*)&cmtj::k_junction_lx<R, L, S, FM, WPE, ND>,       \
+   "k_junction_ll<" #R "," #L "," #S "," #FM "," #ND ",waves " #WPE ">", (ND) + 1}
 
 #define CMTJ_KC(L, FM, ND)                                                                     \
   {CMTJ_FP32, L, 4 * (L), CMTJ_RK4, FM, false, (const void*)&cmtj::k_junction_cl<L, FM, ND>,  \
