@@ -1,4 +1,5 @@
-// Dipole-coupled group kernels: one group per workgroup, one element per
+// Dipole-coupled group kernels of the couplings and features that
+// k_group_cl.hip has no kernel for: one group per workgroup, one element per
 // lane of its first wave (every feature, FP64), the group field of each step
 // built in LDS from the elements' top-layer magnetisations (GroupInteraction,
 // core/reservoir.hpp:121-230).  The reference steps a group with RK4, or

@@ -41,6 +41,7 @@ constexpr int QP_SWAP2 = 0x4E;  // quad_perm [2,3,0,1]
 constexpr int QP_BC0 = 0x00;    // quad_perm [0,0,0,0]: x to every lane of the quad
 constexpr int DPP_ROW_SHR4 = 0x114;  // lane i reads lane i - 4 (0 outside the row)
 constexpr int DPP_ROW_SHL4 = 0x104;  // lane i reads lane i + 4
+constexpr int DPP_HALF_MIRROR = 0x141;  // lane i reads lane 7 - i of its 8
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -290,6 +291,25 @@ __device__ __forceinline__ bool sine_kind(int type) {
   return type == CMTJ_SINE || type == CMTJ_POSINE || type == CMTJ_HALFSINE;
 }
 
+// What the waves of a dipole-coupled group share: the elements' top-layer m
+// scaled by their source strengths, in two copies taken in turn (one barrier
+// a step: a wave writes a copy again only after the barrier of the step
+// between, which every wave reaches with its reads of that copy done), and a
+// word per wave for the decisions the waves take together.
+template <int GW, int EPW>
+struct GroupClLds {
+  alignas(32) double sm[2][GW * EPW][4];
+  uint32_t word[GW];
+};
+
+// The barrier between LDS writes and other waves' reads; global stores in
+// flight (log entries) are not waited for.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ND: number of time-dependent records when fixed at compile time (exact
 // kernels), -1 to read it from the group.  F64: every stage in binary64
 // (the drop-in's arithmetic) instead of the anchored binary32 increments.
@@ -302,6 +322,10 @@ __device__ __forceinline__ bool sine_kind(int type) {
 // from the members' magnetisations at the start of the step and the stack
 // current replaces the members' current at every stage, as in k_junction's
 // stack form (binary64 only).
+// GW: workgroup b of GW waves is dipole-coupled group b (GroupInteraction,
+// core/reservoir.hpp:121-230, Kanao and Nomura coupling; binary64 RK4),
+// element e on the 4L lanes from 4L e, at most GW 64/(4L) elements; the field
+// of the step's other elements joins the frozen terms (see group_field_cl).
 //
 // What bounds it: with at most one wave per SIMD a step takes four cycles per
 // instruction the wave issues (binary64 and binary32 alike, wait states
@@ -316,12 +340,15 @@ __device__ __forceinline__ bool sine_kind(int type) {
 // binary64 steps 21.5 -> 12.5 ms; 512 oscillators x 50,000 steps 44.2 -> 15.4
 // ms; 1023 one-layer instances under a sine field x 10,000 steps 14.9 -> 3.1
 // ms (three binary64 sines a step before, see Osc).
-template <int L, uint32_t FM, int ND, bool F64 = false, int SOLVER = CMTJ_RK4, int LOGF = 0, bool STK = false>
-__global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
+template <int L, uint32_t FM, int ND, bool F64 = false, int SOLVER = CMTJ_RK4, int LOGF = 0, bool STK = false,
+          int GW = 0>
+__global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArgs g) {
   // the compiled-in layout's R is layer 0 against layer 1
   static_assert(LOGF == 0 || (L == 2 && (FM & F_EXACT) && (FM & F_IEC)), "two coupled layers");
   static_assert(!STK || (F64 && LOGF == 0 && !(FM & F_KSTEP)),
                 "stacks: binary64, the group's log layout, every step through the same code");
+  static_assert(GW == 0 || (F64 && SOLVER == CMTJ_RK4 && LOGF == 0 && !STK && L <= 2 && !(FM & F_KSTEP)),
+                "groups: binary64 RK4, the group's log layout, every step through the same code");
   static_assert(L == 1 || L == 2 || L == 4, "4L lanes per instance must divide a 16-lane DPP row");
   static_assert(F64 || !(FM & (F_STT | F_SOT | F_SOT2 | F_DYN | F_THERMAL | F_ANIS2 | F_IEC2 | F_DEMAG_OFF |
                                 F_IDMI | F_DIPOLE)),
@@ -339,7 +366,21 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
   int q;
   [[maybe_unused]] const cmtj_stack* sk = nullptr;
   [[maybe_unused]] int s_j = 0, s_n = 0, s_base = 0, s_lane0 = 0;
-  if constexpr (STK) {
+  [[maybe_unused]] const cmtj_group* gp = nullptr;
+  [[maybe_unused]] int g_n = 0, g_e = 0, g_top = 0;
+  bool own = true;  // the lanes hold an instance
+  if constexpr (GW > 0) {
+    // every lane stays for the barriers and lane moves: lanes past the
+    // group's elements hold an element without layers (m = 0, strength 0)
+    if (blockIdx.x >= g.group_n) return;
+    gp = g.group + blockIdx.x;
+    g_n = gp->n_elements;
+    g_e = (int)(threadIdx.x / LPI);
+    own = g_e < g_n;
+    inst = blockIdx.x * (uint32_t)g_n + (uint32_t)(own ? g_e : 0);
+    q = (int)(threadIdx.x % LPI);
+    g_top = own ? gp->top[g_e] : 0;
+  } else if constexpr (STK) {
     // lanes of a stack past its members leave at once; a stack never
     // straddles a wave (pad is a power of two of at most 64)
     const uint32_t pad = g.stack_pad, sid = gl / pad;
@@ -360,7 +401,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
   const int ly = q >> 2, c = q & 3;
   const uint32_t fl = g.flags;
   const int nl = g.nl;
-  const bool lact = ly < nl;          // the lane's layer exists
+  const bool lact = own && ly < nl;   // the lane's layer exists
   const bool live = lact && c < 3;    // the lane holds a component
   const int lyr = lact ? ly : 0;
   const uint32_t jid = g.order[inst];
@@ -561,7 +602,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
   // store: the m channels on the lanes of their components, R on a lane that
   // writes no m (compiled-in layout: the y lane of layer 0; else layer 0's
   // pad lane, which takes it from the x lane)
-  const bool rlane = classic && q == (LOGF == 1 ? 1 : 3);
+  const bool rlane = own && classic && q == (LOGF == 1 ? 1 : 3);
   const bool wlog = wm || rlane;
   char* const lpl = lp + (rlane ? orr : om);  // the lane's entry 0
   // STRIP coefficients of the lane's layer, read once (the descriptors may
@@ -624,6 +665,107 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
     const V3<double> pv = mk<double>(sl.pol[0], sl.pol[1], sl.pol[2]);
     s_pol = {comp(pv, c), comp(pv, c1), comp(pv, c2)};
   }
+
+  // Groups: field of the other elements on this lane's component of its
+  // element's top layer, from the start-of-step m (stepFunctionalSolver,
+  // core/reservoir.hpp:126-147),
+  //   sum_j s_j (3 (m_j . r) r / |r|^5 - m_j / |r|^3),  r = r_e - r_j,
+  // s_j = (Ms_j / mu0) V_j (computeDipoleInteraction, :79-96) or Ms_j V_j /
+  // mu0 / (4 pi) (computeDipoleInteractionNoumra, :106-119).  The geometry is
+  // constant, so a lane keeps each of its pairs as four numbers, u = r
+  // sqrt(3 / |r|^5) and w = 1 / |r|^3, and a pair costs nine FMAs on s_j m_j
+  // from LDS: u (u . sm) - w sm.  The eight lanes of an octet take the
+  // sources j = o (mod 8); with one-layer elements an octet is two elements
+  // and a lane sums its sources for both (each source read once: with one
+  // element a lane, reading the sources took longer than the FMAs).  The
+  // octet's sums meet by lane moves, component c ends in lane c.
+  constexpr int GS = (GW > 0) ? GW * (64 / LPI) / 8 : 1;  // sources per lane
+  constexpr int GP = (L == 1) ? 2 : 1;                    // elements per octet
+  [[maybe_unused]] Rot<double> gu[GP][GS];
+  [[maybe_unused]] double gw[GP][GS];
+  [[maybe_unused]] double g_s = 0.0;
+  [[maybe_unused]] int g_buf = 0;
+  [[maybe_unused]] bool g_lane = false, g_sink = false;  // the lane holds a component of the top layer; its m
+  __shared__ GroupClLds<(GW > 0 ? GW : 1), (GW > 0 ? 64 / LPI : 1)> glds;
+  if constexpr (GW > 0) {
+    g_lane = live && ly == g_top;
+    g_sink = c < 3 && ly == g_top;
+    const int o = (int)(threadIdx.x & 7u);
+    if (g_lane) {
+      const cmtj_layer& Ly = g.layers[J->layer_offset + g_top];
+      const double V = Ly.thickness * Ly.cell_surface;
+      g_s = (gp->interaction == CMTJ_INTERACTION_KANAO)    ? (Ly.Ms / g.c.mu0) * V
+            : (gp->interaction == CMTJ_INTERACTION_NOMURA) ? Ly.Ms * V / g.c.mu0 / (4 * M_PI)
+                                                           : 0.0;  // nullDipoleInteraction
+    }
+#pragma unroll
+    for (int p = 0; p < GP; ++p) {
+      const int e = (p == 0) ? g_e : (g_e ^ 1);
+#pragma unroll
+      for (int s = 0; s < GS; ++s) {
+        const int j = 8 * s + o;
+        const bool on = e < g_n && j < g_n && j != e;
+        const int ei = on ? e : 0, ji = on ? j : 0;
+        const double dx = gp->pos[ei][0] - gp->pos[ji][0], dy = gp->pos[ei][1] - gp->pos[ji][1],
+                     dz = gp->pos[ei][2] - gp->pos[ji][2];
+        // the host has checked |r| against the reference's limits
+        const double il = on ? 1.0 / sqrt(dx * dx + dy * dy + dz * dz) : 0.0, il2 = il * il;
+        const double f = sqrt(3.0 * (il2 * il)) * il;
+        gu[p][s] = {dx * f, dy * f, dz * f};
+        gw[p][s] = il2 * il;
+      }
+    }
+  }
+  auto group_field_cl = [&]() __attribute__((always_inline)) -> double {
+    if constexpr (GW > 0) {
+      auto& sm = glds.sm[g_buf];
+      g_buf ^= 1;
+      if (g_sink) sm[g_e][c] = g_s * m.a;
+      lds_barrier();
+      V3<double> acc[GP];
+#pragma unroll
+      for (int p = 0; p < GP; ++p) acc[p] = mk<double>(0, 0, 0);
+      const int o = (int)(threadIdx.x & 7u);
+#pragma unroll
+      for (int s = 0; s < GS; ++s) {
+        const double x = sm[8 * s + o][0], y = sm[8 * s + o][1], z = sm[8 * s + o][2];
+#pragma unroll
+        for (int p = 0; p < GP; ++p) {
+          const Rot<double>& u = gu[p][s];
+          const double d = fma(u.c, z, fma(u.b, y, u.a * x)), w = -gw[p][s];
+          acc[p].x = fma(u.a, d, fma(w, x, acc[p].x));
+          acc[p].y = fma(u.b, d, fma(w, y, acc[p].y));
+          acc[p].z = fma(u.c, d, fma(w, z, acc[p].z));
+        }
+      }
+      V3<double> h = acc[0];
+      h.x += dpp_d<DPP_HALF_MIRROR>(acc[GP - 1].x);
+      h.y += dpp_d<DPP_HALF_MIRROR>(acc[GP - 1].y);
+      h.z += dpp_d<DPP_HALF_MIRROR>(acc[GP - 1].z);
+      // over the quad: lanes 0, 1 gather x and y, lanes 2, 3 gather z
+      const bool up = c >= 2;
+      const double a = (up ? h.z : h.x) + dpp_d<QP_SWAP2>(up ? h.x : h.z);
+      const double b = h.y + dpp_d<QP_SWAP2>(h.y);
+      const double r = (c == 1 ? b : a) + dpp_d<QP_SWAP1>(c == 0 ? b : a);
+      return g_lane ? K.g * r : 0.0;
+    } else {
+      return 0.0;
+    }
+  };
+  // whether any wave of the group says so (every wave calls it; the next
+  // step's barrier lies before the next write)
+  auto group_any = [&](bool mine) __attribute__((always_inline)) -> bool {
+    if constexpr (GW > 1) {
+      glds.word[threadIdx.x >> 6] = mine ? 1u : 0u;
+      lds_barrier();
+      uint32_t any = 0;
+#pragma unroll
+      for (int w = 0; w < GW; ++w) any |= glds.word[w];
+      return __builtin_amdgcn_readfirstlane(any) != 0u;
+    } else {
+      return mine;
+    }
+  };
 
   // Value of record r at the present stage time (ts): sine kinds from their
   // carried phase, the others from the waveform.
@@ -707,6 +849,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
   // run stops on it have taken the step (their m as the reference leaves
   // it); the others left their state alone and take the step again.
   unsigned long long hitb = 0ull;
+  [[maybe_unused]] bool hitg = false;  // groups: a NaN in any wave of the group
   double dev = 0.0;
   uint64_t next_log = 0;   // LOGM 0: step of the next entry
   char* pk = lpl;          // the lane's next entry
@@ -737,6 +880,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
       }
       stack_current(sl, s_j, s_n, s_base, LPI, dq, t, dt, g.tables, i, sI, sIlog, sClog);
     }
+    [[maybe_unused]] const double gH = group_field_cl();
     // ---- drives at ts: this component's field slots and the layer's scalar
     // slots (the slot of a record is wave-uniform: one scalar branch)
     auto route = [&](CLDrive& d, int meta, bool on, double v) __attribute__((always_inline)) {
@@ -794,7 +938,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
     // frozen neighbours' terms (IEC, :654-675; IDMI, :677-693; dipole
     // tensors, :579-586, with this layer's Ms)
     auto frozen = [&](const CLDrive& d, const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> Rot<double> {
-      if constexpr (!DRIVEN && !DYNS && !(FM & (F_IDMI | F_DIPOLE))) {
+      if constexpr (!DRIVEN && !DYNS && !(FM & (F_IDMI | F_DIPOLE)) && GW == 0) {
         // constant field and coupling: the neighbours' components are in the lane
         Rot<double> B{K.hb, K.hb1, K.hb2};
         if (CMTJ_HAS(F_IEC)) {
@@ -804,7 +948,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
         }
         return B;
       }
-      double b = d.H;
+      double b = (GW > 0) ? d.H + gH : d.H;
 #pragma unroll
       for (int n = 0; n < NN; ++n) {
         if (CMTJ_HAS(F_IEC) || CMTJ_HAS(F_IEC2)) b = fma(nbs[n].a, DYNS ? d.J[n] * K.ginv_mst : K.jn[n], b);
@@ -1019,15 +1163,17 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
     if constexpr (CHK) {
       const unsigned long long bad = __ballot(isnan(mnew.a)) & nan_lanes;
       hitb = bad;
-      if (__builtin_expect(bad != 0ull, 0)) {
+      if constexpr (GW > 0) hitg = group_any(bad != 0ull);
+      if (__builtin_expect((GW > 0) ? hitg : bad != 0ull, 0)) {
         // a NaN in the wave (rare): layers up to and including the instance's
         // first NaN layer take the new value; a member's NaN ends its stack's
-        // run (the reference throws), the other members take this step and
-        // stop with it (selects, no per-lane branch: the whole test stays
+        // or group's run (the reference throws), the other members take this
+        // step and stop with it (selects, no per-lane branch: the whole test stays
         // wave-uniform)
         const uint32_t gb = (uint32_t)((bad >> gshift) & ((1ull << LPI) - 1));
         bool take = (gb != 0u) & (ly <= (int)(__builtin_ctz(gb | 0x80000000u) >> 2));
         if constexpr (STK) take = take | ((gb == 0u) & ((bad & s_mask) != 0ull));
+        if constexpr (GW > 0) take = take | (gb == 0u);
         m.a = take ? mnew.a : m.a;
         return;
       }
@@ -1054,7 +1200,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
           rx += __shfl_xor(rx, o, 64);
           ry += __shfl_xor(ry, o, 64);
         }
-        if (q == 0) {
+        if (own && q == 0) {
           log_put(f32log, pk - om + orr, 1 / rx);
           log_put(f32log, pk - om + orr + cs, 1 / ry);
         }
@@ -1195,6 +1341,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
                 k += ne;
               }
               redo = __ballot(!(dev <= kUnitRange * kUnitRange)) != 0ull;
+              if constexpr (GW > 0) redo = group_any(redo);
               slow = (redo && flagged) ? 31u : 0u;
               flagged = redo;
               if (redo) {
@@ -1213,7 +1360,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
               for (uint32_t u = u0; u < ue; ++u) {
                 i = i0 + u;
                 step(drv_tag, I0{}, std::true_type{});
-                if (hitb) {
+                if ((GW > 0) ? hitg : hitb != 0ull) {
                   end = u;
                   break;
                 }
@@ -1228,10 +1375,11 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
           u0 = ue;
         }
         i = i0 + end;
-        if (hitb) {
+        if ((GW > 0) ? hitg : hitb != 0ull) {
           const uint32_t gb = (uint32_t)((hitb >> gshift) & ((1ull << LPI) - 1));
           bool stop = gb != 0u;
           if constexpr (STK) stop = stop || (hitb & s_mask) != 0ull;
+          if constexpr (GW > 0) stop = true;
           if (gb) {
             nan_layer = __builtin_ctz(gb) >> 2;
             code = CMTJ_ERR_NAN;
@@ -1267,7 +1415,7 @@ __global__ __launch_bounds__(64) void k_junction_cl(GroupArgs g) {
     phase(iend, std::true_type{});
   }
   if (g.mag_out && live) g.mag_out[((size_t)jid * CMTJ_MAX_LAYERS + ly) * 3 + c] = m.a;
-  if (g.status && q == 0) {
+  if (g.status && own && q == 0) {
     cmtj_status s;
     s.code = code;
     s.steps_done = i;

@@ -8,7 +8,7 @@ namespace cmtj {
 struct KEntry {
   int prec;
   int lm;   // layer capacity
-  int lpi;  // lanes per instance: 1 (k_junction), lm (k_junction_ll) or 4 lm (k_junction_cl)
+  int lpi;  // lanes per instance: 1 (k_junction), lm (k_junction_ll) or 4 lm (k_junction_cl); kernels_group_cl: elements
   int solver;
   uint32_t fm;
   bool loge;
@@ -32,6 +32,7 @@ constexpr uint32_t FM_SOTT = F_ANIS | F_IEC | F_DYN | F_DYNH | F_SOT | F_THERMAL
 constexpr uint32_t FM_STTC = F_ANIS | F_ANIS2 | F_IEC | F_IEC2 | F_DEMAG_OFF | F_IDMI | F_DIPOLE | F_DYNH | F_DYN |
                              F_STT | F_SOT | F_SOT2;
 // coupled runs (stacks, groups): the usual member's features
+constexpr uint32_t FM_STATIC = F_ANIS | F_IEC;  // the lean set under constant drives
 constexpr uint32_t FM_CPL = F_ANIS | F_IEC | F_DYN | F_DYNH | F_STT | F_SOT | F_THERMAL;
 
 // exact feature sets of the benchmark workloads (see workloads.py)
@@ -60,6 +61,7 @@ const void* dp_queue_kernel();   // single-layer Dormand-Prince from a device wo
 const void* clear_u32_kernel();  // clears a launch's work counters
 KTable kernels_group();   // dipole-coupled groups, one wave each: chosen by cmtj_run_groups only
 KTable kernels_group4();  // the same on four waves per group
+KTable kernels_group_cl();  // Kanao / Nomura groups on one lane per component
 
 }  // namespace cmtj
 
@@ -96,6 +98,12 @@ KTable kernels_group4();  // the same on four waves per group
 #define CMTJ_KC64H(L, FM, ND)                                                                      \
   {CMTJ_FP64, L, 4 * (L), CMTJ_HEUN, FM, false, (const void*)&cmtj::k_junction_cl<L, FM, ND, true, CMTJ_HEUN>, \
    "k_junction_cl<double," #L ",Heun," #FM "," #ND ">", (ND) + 1}
+
+// dipole-coupled groups of at most GW 64 / (4L) elements
+#define CMTJ_KGC(L, FM, GW)                                                                                        \
+  {CMTJ_FP64, L, (GW) * 64 / (4 * (L)), CMTJ_RK4, FM, false,                                                       \
+   (const void*)&cmtj::k_junction_cl<L, FM, -1, true, CMTJ_RK4, 0, false, GW>,                                     \
+   "k_junction_cl<double," #L "," #FM ",group of " #GW " waves>"}
 
 #define CMTJ_KL_SOLVERS(R, PREC, L, FM) \
   CMTJ_KL(R, PREC, L, CMTJ_RK4, FM), CMTJ_KL(R, PREC, L, CMTJ_HEUN, FM), CMTJ_KL(R, PREC, L, CMTJ_EULER_HEUN, FM)
