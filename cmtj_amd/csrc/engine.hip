@@ -6,6 +6,8 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
@@ -286,6 +288,7 @@ struct Group {
   GroupArgs a;
   uint32_t blocks;
   uint32_t threads = 64;  // per workgroup
+  uint32_t steps = 0;     // of its longest instance (Dormand-Prince: at least)
   uint32_t* queue = nullptr;  // work counter of a queue launch (k_dp_q), else null
 };
 
@@ -479,6 +482,7 @@ static int build_plan(cmtj_plan* P, const cmtj_junction* js, size_t n, const cmt
     for (size_t q = 0; q < r0.size(); ++q) Gr.a.dmeta[q] = r0[q].meta;
     Gr.a.c = *c;
     Gr.blocks = (uint32_t)(((uint64_t)Gr.a.n * (uint64_t)k->lpi + 63) / 64);
+    Gr.steps = j0.n_steps;  // longest first
     if (lanes == CMTJ_LANES_QUEUE && j0.solver == CMTJ_DORMAND_PRINCE && j0.n_layers == 1) {
       Gr.queue = (uint32_t*)(arena + o_queue) + g;
       Gr.blocks = (std::min<uint32_t>(Gr.a.n, queue_lanes()) + 63) / 64;
@@ -508,9 +512,11 @@ static int build_plan(cmtj_plan* P, const cmtj_junction* js, size_t n, const cmt
   return 0;
 }
 
+// Launches every group of a plan: on s, group q on streams[q % n_streams], or
+// (lane_of) group q on streams[lane_of[q]].
 static int launch_plan(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_status, hipStream_t s,
                        cmtj_state* d_state = nullptr, uint32_t slice = 0, void* const* streams = nullptr,
-                       int n_streams = 0) {
+                       int n_streams = 0, const int* lane_of = nullptr) {
   g_last_kernels.clear();
   for (size_t q = 0; q < P->groups.size(); ++q) {
     Group& G = P->groups[q];
@@ -522,7 +528,8 @@ static int launch_plan(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_
     a.state = d_state;
     a.slice = slice;
     void* args[] = {&a};
-    const hipStream_t st = n_streams > 0 ? (hipStream_t)streams[q % (size_t)n_streams] : s;
+    const hipStream_t st = n_streams > 0 ? (hipStream_t)streams[lane_of ? (size_t)lane_of[q] : q % (size_t)n_streams]
+                                         : s;
     if (G.queue) {
       uint32_t* ctr = G.queue;
       uint32_t one = 1;
@@ -536,6 +543,169 @@ static int launch_plan(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_
   }
   return 0;
 }
+
+// ---------------------------------------------------------------------------
+// Groups side by side.  A batch of requests falls into groups of a few waves
+// each whose launches, one after another on the caller's stream, leave most
+// of the chip idle: its time is the sum of the groups' longest runs.  They
+// share nothing but read-only descriptors, so an execute forks the small ones
+// onto side streams and joins them before it returns: the caller's stream
+// order is that of one launch.
+
+namespace {
+constexpr int kSideStreams = 3;  // with the caller's stream the four hardware queues of a process
+constexpr int kSideSets = 4;     // per device
+
+// Streams and events of one fork.  A set is taken for the enqueueing of one
+// execute and reused only when the work last put on it is done (otherwise one
+// caller's groups would wait for another's, whose streams may wait for
+// anything); with every set in use the launches follow one another.
+struct SideSet {
+  hipStream_t stream[kSideStreams] = {};
+  hipEvent_t fork = nullptr, join[kSideStreams] = {};
+  bool used[kSideStreams] = {};  // the joins of the last execute
+  bool taken = false;
+};
+struct SidePool {
+  std::mutex mu;
+  std::map<int, std::vector<std::unique_ptr<SideSet>>> sets;  // by device; kept to the end of the process
+};
+SidePool& side_pool() {
+  static SidePool* p = new SidePool;  // (never destroyed: streams must not outlive the runtime's own teardown)
+  return *p;
+}
+
+// queries and stream creation are barred on a thread while another thread
+// captures globally, unless its own mode is relaxed
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+bool make_set(SideSet& t) {
+  bool ok = hipEventCreateWithFlags(&t.fork, hipEventDisableTiming) == hipSuccess;
+  for (int q = 0; ok && q < kSideStreams; ++q)
+    ok = hipStreamCreateWithFlags(&t.stream[q], hipStreamNonBlocking) == hipSuccess &&
+         hipEventCreateWithFlags(&t.join[q], hipEventDisableTiming) == hipSuccess;
+  if (ok) return true;
+  (void)hipGetLastError();
+  for (int q = 0; q < kSideStreams; ++q) {
+    if (t.join[q]) (void)hipEventDestroy(t.join[q]);
+    if (t.stream[q]) (void)hipStreamDestroy(t.stream[q]);
+  }
+  if (t.fork) (void)hipEventDestroy(t.fork);
+  return false;
+}
+
+SideSet* take_set() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  const RelaxedCapture relaxed;
+  SidePool& pool = side_pool();
+  std::lock_guard<std::mutex> lk(pool.mu);
+  auto& v = pool.sets[dev];
+  for (auto& t : v) {
+    if (t->taken) continue;
+    bool idle = true;
+    for (int q = 0; q < kSideStreams && idle; ++q)
+      if (t->used[q] && hipEventQuery(t->join[q]) != hipSuccess) {
+        (void)hipGetLastError();  // not ready is no error of the caller's
+        idle = false;
+      }
+    if (idle) {
+      t->taken = true;
+      return t.get();
+    }
+  }
+  if (v.size() >= (size_t)kSideSets) return nullptr;
+  std::unique_ptr<SideSet> t(new SideSet);
+  if (!make_set(*t)) return nullptr;
+  t->taken = true;
+  v.push_back(std::move(t));
+  return v.back().get();
+}
+
+struct GiveBack {
+  void operator()(SideSet* t) const {
+    std::lock_guard<std::mutex> lk(side_pool().mu);
+    t->taken = false;
+  }
+};
+
+// Which stream each group of an execute takes (0: the caller's): groups that
+// fill the chip stay on the caller's, the others go to the least loaded one,
+// longest first.  False where the fork is not worth its events: less than
+// 1000 steps run beside the longest stream, some 0.2 ms at 0.2 us per step,
+// against about 0.03 ms for the events.
+bool spread_groups(const cmtj_plan& P, std::vector<int>& lane_of) {
+  const size_t G = P.groups.size();
+  lane_of.assign(G, 0);
+  if (G < 2) return false;
+  uint64_t load[1 + kSideStreams] = {}, total = 0;
+  std::vector<size_t> small;
+  for (size_t q = 0; q < G; ++q) {
+    const Group& g = P.groups[q];
+    total += g.steps;
+    if ((uint64_t)g.blocks * (g.threads / 64) >= 2 * kSimds)
+      load[0] += g.steps;
+    else
+      small.push_back(q);
+  }
+  std::stable_sort(small.begin(), small.end(), [&](size_t a, size_t b) { return P.groups[a].steps > P.groups[b].steps; });
+  for (size_t q : small) {
+    const int t = (int)(std::min_element(load, load + 1 + kSideStreams) - load);
+    lane_of[q] = t;
+    load[t] += P.groups[q].steps;
+  }
+  return total - *std::max_element(load, load + 1 + kSideStreams) >= 1000;
+}
+
+// Launches the plan's groups side by side, ordered on s as one launch would be.
+int launch_spread(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_status, hipStream_t s) {
+  std::vector<int> lane_of;
+  std::unique_ptr<SideSet, GiveBack> t;
+  if (spread_groups(*P, lane_of)) {
+    // a capturing stream keeps the launches on itself: forked streams would
+    // stay part of the capture until it ends
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess)
+      (void)hipGetLastError();
+    else if (cap == hipStreamCaptureStatusNone)
+      t.reset(take_set());
+    if (t && hipEventRecord(t->fork, s) != hipSuccess) {  // a stream of another device, say: as without the fork
+      (void)hipGetLastError();
+      t.reset();
+    }
+  }
+  if (!t) return launch_plan(P, d_log, d_mag, d_status, s);
+  void* streams[1 + kSideStreams] = {(void*)s};
+  bool used[kSideStreams] = {};
+  for (int l : lane_of)
+    if (l > 0) used[l - 1] = true;
+  hipError_t e = hipSuccess;
+  for (int q = 0; q < kSideStreams; ++q) {
+    streams[1 + q] = (void*)t->stream[q];
+    if (e == hipSuccess && used[q]) e = hipStreamWaitEvent(t->stream[q], t->fork, 0);
+  }
+  int r = 0;
+  if (e == hipSuccess)
+    r = launch_plan(P, d_log, d_mag, d_status, s, nullptr, 0, streams, 1 + kSideStreams, lane_of.data());
+  // joined also after a failed launch: what did start stays ordered on s
+  for (int q = 0; q < kSideStreams; ++q) {
+    if (!used[q]) continue;
+    hipError_t j = hipEventRecord(t->join[q], t->stream[q]);
+    if (j == hipSuccess) {
+      t->used[q] = true;
+      j = hipStreamWaitEvent(s, t->join[q], 0);
+    }
+    if (e == hipSuccess) e = j;
+  }
+  if (r) return r;
+  HIP_TRY(e);
+  return 0;
+}
+}  // namespace
 
 // ---------------------------------------------------------------------------
 // the drop-in context: one stream, grow-only device buffers
@@ -1206,7 +1376,7 @@ int cmtj_plan_execute(cmtj_plan* p, void* d_log, size_t log_capacity, double* d_
   if (d_log && log_capacity < p->log_extent)
     return fail(CMTJ_ERR_INVALID, "log buffer smaller than the plan's log extent (" +
                                       std::to_string(p->log_extent) + " elements)");
-  return launch_plan(p, d_log, d_mag_out, d_status, (hipStream_t)stream);
+  return launch_spread(p, d_log, d_mag_out, d_status, (hipStream_t)stream);
 }
 
 int cmtj_plan_execute_slice(cmtj_plan* p, void* d_log, size_t log_capacity, double* d_mag_out,
