@@ -557,7 +557,8 @@ constexpr int kSideStreams = 3;  // with the caller's stream the four hardware q
 constexpr int kSideSets = 4;     // per device
 
 // Streams and events of one fork.  A set is taken for the enqueueing of one
-// execute and reused only when the work last put on it is done (otherwise one
+// execute and reused for the same caller's stream, whose order its joins are
+// part of already, or when the work last put on it is done (otherwise one
 // caller's groups would wait for another's, whose streams may wait for
 // anything); with every set in use the launches follow one another.
 struct SideSet {
@@ -565,6 +566,7 @@ struct SideSet {
   hipEvent_t fork = nullptr, join[kSideStreams] = {};
   bool used[kSideStreams] = {};  // the joins of the last execute
   bool taken = false;
+  hipStream_t user = nullptr;  // the caller's stream of the last execute
 };
 struct SidePool {
   std::mutex mu;
@@ -598,13 +600,18 @@ bool make_set(SideSet& t) {
   return false;
 }
 
-SideSet* take_set() {
+SideSet* take_set(hipStream_t s) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   const RelaxedCapture relaxed;
   SidePool& pool = side_pool();
   std::lock_guard<std::mutex> lk(pool.mu);
   auto& v = pool.sets[dev];
+  for (auto& t : v)
+    if (!t->taken && t->user == s) {
+      t->taken = true;
+      return t.get();
+    }
   for (auto& t : v) {
     if (t->taken) continue;
     bool idle = true;
@@ -614,6 +621,7 @@ SideSet* take_set() {
         idle = false;
       }
     if (idle) {
+      t->user = s;
       t->taken = true;
       return t.get();
     }
@@ -621,6 +629,7 @@ SideSet* take_set() {
   if (v.size() >= (size_t)kSideSets) return nullptr;
   std::unique_ptr<SideSet> t(new SideSet);
   if (!make_set(*t)) return nullptr;
+  t->user = s;
   t->taken = true;
   v.push_back(std::move(t));
   return v.back().get();
@@ -672,7 +681,7 @@ int launch_spread(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_statu
     if (hipStreamIsCapturing(s, &cap) != hipSuccess)
       (void)hipGetLastError();
     else if (cap == hipStreamCaptureStatusNone)
-      t.reset(take_set());
+      t.reset(take_set(s));
     if (t && hipEventRecord(t->fork, s) != hipSuccess) {  // a stream of another device, say: as without the fork
       (void)hipGetLastError();
       t.reset();
