@@ -112,17 +112,25 @@ static const KEntry* pick_kernel(int prec, int nl, int solver, uint32_t flags, u
   // (spin torques, scalar drives), it stands in for the missing binary32
   // one: more accurate, and on batches that leave SIMDs idle faster than
   // binary32 one lane per layer (a 512-point STO sweep: 5.9e8 vs 3.2e8
-  // junction-steps/s).  Not for Euler-Heun: its binary64 normals cost more
-  // than the binary32 ones of one lane per layer.
+  // junction-steps/s).  Stochastic solvers have their own
+  // there, with binary32 normals.
   if (!best[2] && cl64) best[2] = cl64;
   if (lanes == CMTJ_LANES_ONE && best[0]) return best[0];
-  if (lanes == CMTJ_LANES_PER_COMPONENT && best[2]) return best[2];
+  // (FP32 Euler-Heun and Heun take it by the automatic choice only: a caller
+  // that asks for components runs them per layer at every size, so that a
+  // server's groups may fill the chip: 65,536 switching devices 0.9 us per
+  // step per layer, 2.3 us per component)
+  const bool noise32 = prec == CMTJ_FP32 && solver != CMTJ_RK4;
+  if (lanes == CMTJ_LANES_PER_COMPONENT && best[2] && !noise32) return best[2];
   // automatic choice: on a batch too small to fill the chip, the time of a
   // sweep is its longest instance's step count times the latency of one
   // wave step.  One lane per component issues about half the instructions
   // per wave step of one lane per layer (111 against 199 VALU on the PIMM
   // set), at four times the lanes: it wins while its waves still fit one per
-  // SIMD, and costs about twice the instructions per junction-step beyond that.
+  // SIMD, and costs about twice the instructions per junction-step beyond that
+  // (FP32 Euler-Heun, us per step: 8,192 two-layer switching devices 0.41
+  // against 0.53, 16,384 0.65 against 0.55; 4,096 four-layer chains 0.90
+  // against 1.09, 8,192 1.74 against 1.18).
   if (lanes == CMTJ_LANES_AUTO && best[2] && n_inst * (uint64_t)best[2]->lpi <= 64 * kSimds) return best[2];
   // one lane per layer for multilayer instances: its register footprint is
   // smaller than one lane per instance's, so more waves fit per SIMD, and the

@@ -39,6 +39,7 @@ constexpr int QP_ROT2 = 0xD2;   // quad_perm [2,0,1,3]: component c reads c + 2 
 constexpr int QP_SWAP1 = 0xB1;  // quad_perm [1,0,3,2]
 constexpr int QP_SWAP2 = 0x4E;  // quad_perm [2,3,0,1]
 constexpr int QP_BC0 = 0x00;    // quad_perm [0,0,0,0]: x to every lane of the quad
+constexpr int QP_NEXT = 0x39;   // quad_perm [1,2,3,0]: the quad's values move down one lane
 constexpr int DPP_ROW_SHR4 = 0x114;  // lane i reads lane i - 4 (0 outside the row)
 constexpr int DPP_ROW_SHL4 = 0x104;  // lane i reads lane i + 4
 constexpr int DPP_HALF_MIRROR = 0x141;  // lane i reads lane 7 - i of its 8
@@ -253,7 +254,7 @@ struct CLConst {
   // coefficients; secondary SOT: g, g alpha
   double sta, stb, num, lam, lam2, wc;
   double ga, gaa, dlt, flt, g2, g2a;
-  double sig2, gconv;             // 2 alpha kB / (Ms V gamma), -gamma / (1 + alpha^2)
+  double sig2, kick, sg0;         // 2 alpha kB / (Ms V gamma), -gamma / (1 + alpha^2) sqrt(dt), kick sqrt(sig2 T)
   bool stt, alt, dyn_sot, stat_i, therm;  // STT; its alternative form; SOT from drivers; current-driven torque; thermal
 };
 
@@ -341,12 +342,13 @@ __device__ __forceinline__ void lds_barrier() {
 // ms; 1023 one-layer instances under a sine field x 10,000 steps 14.9 -> 3.1
 // ms (three binary64 sines a step before, see Osc).
 template <int L, uint32_t FM, int ND, bool F64 = false, int SOLVER = CMTJ_RK4, int LOGF = 0, bool STK = false,
-          int GW = 0>
+          int GW = 0, bool NF = false>
 __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArgs g) {
   // the compiled-in layout's R is layer 0 against layer 1
   static_assert(LOGF == 0 || (L == 2 && (FM & F_EXACT) && (FM & F_IEC)), "two coupled layers");
   static_assert(!STK || (F64 && LOGF == 0 && !(FM & F_KSTEP)),
                 "stacks: binary64, the group's log layout, every step through the same code");
+  static_assert(!NF || (F64 && SOLVER != CMTJ_RK4 && (FM & F_THERMAL)), "binary32 normals: stochastic solvers");
   static_assert(GW == 0 || (F64 && SOLVER == CMTJ_RK4 && LOGF == 0 && !STK && L <= 2 && !(FM & F_KSTEP)),
                 "groups: binary64 RK4, the group's log layout, every step through the same code");
   static_assert(L == 1 || L == 2 || L == 4, "4L lanes per instance must divide a 16-lane DPP row");
@@ -419,7 +421,6 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   const double Rp = J->Rp, Rap = J->Rap;
   [[maybe_unused]] const double hR = (Rap - Rp) / 2.0;
   [[maybe_unused]] const uint64_t seed = J->seed, stream = J->stream;
-  [[maybe_unused]] const double sdt = sqrt(dt);
   constexpr int sps = 3;
   const bool hasB = lact && ly > 0, hasT = lact && ly + 1 < nl;
   // whether neighbour n exists, and whether it is the top one (L = 2: the
@@ -496,7 +497,6 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     K.ref = {live ? comp(r1, c) : z, live ? comp(r1, c1) : z, live ? comp(r1, c2) : z};
     K.ref2 = {live ? comp(r2, c) : z, live ? comp(r2, c1) : z, live ? comp(r2, c2) : z};
     K.sig2 = P.sig2;
-    K.gconv = P.gconv;
     const int bits = g.lbits[lyr];
     const int rt = bits & 3;
     const bool sot = live && ((bits >> 2) & 3) == 2;
@@ -532,6 +532,8 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     K.bFL2 = K.dyn_sot ? K.bFL2 : z;
     K.bDL2 = K.dyn_sot ? K.bDL2 : z;
     K.therm = live && ((bits >> 6) & 1) != 0;
+    K.kick = P.gconv * sqrt(dt);
+    K.sg0 = K.therm ? sqrt(K.sig2 * K.bT) * K.kick : z;
   }
   // eta's denominator is lam2 + 1 on every STT lane of the wave (lambda = 1,
   // the usual spacer): the torque then needs no division
@@ -586,6 +588,43 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       sel[k] = false;
     }
   }
+  // whether a drive moves a temperature (else the noise strength is sg0)
+  [[maybe_unused]] bool t_driven = false;
+  if constexpr (DYNS && (FM & F_THERMAL)) {
+#pragma unroll
+    for (int k = 0; k < DREG; ++k)
+      if (k < NR && (ND >= 0 || k < g.ndyn)) t_driven |= ((g.dmeta[k] >> 8) & 0xff) == CMTJ_SLOT_TEMPERATURE;
+    for (int r = DREG; ND < 0 && !(FM & F_EXACT) && r < g.ndyn; ++r)
+      t_driven |= ((g.dmeta[r] >> 8) & 0xff) == CMTJ_SLOT_TEMPERATURE;
+  }
+  // The layer's normals of four steps at a time: lane c of the quad draws
+  // those of step i + c (counter-based, so any lane can), and the step in turn
+  // is read from lane 0, the others moving down.  A draw is most of a
+  // stochastic step's instructions (650 of 840 in binary64), and the quad's
+  // lanes would otherwise all make the same one.  NF: binary32 normals, those
+  // of the other FP32 kernels.
+  using NT = typename std::conditional<NF, float, double>::type;
+  [[maybe_unused]] V3<NT> xi = mk<NT>(0, 0, 0);
+  auto draw = [&](uint32_t step0) __attribute__((always_inline)) {
+    if constexpr (SOLVER != CMTJ_RK4) {
+      if (CMTJ_HAS(F_THERMAL)) xi = thermal_normals<NT>(seed, stream, step0 + (uint32_t)c, (uint32_t)lyr);
+    }
+  };
+  auto next_normals = [&]() __attribute__((always_inline)) -> Rot<double> {
+    auto move = [](auto tag, NT v) __attribute__((always_inline)) -> NT {
+      constexpr int CTRL = decltype(tag)::value;
+      if constexpr (NF)
+        return dpp_f<CTRL>(v);
+      else
+        return dpp_d<CTRL>(v);
+    };
+    constexpr std::integral_constant<int, QP_BC0> BC{};
+    constexpr std::integral_constant<int, QP_NEXT> NX{};
+    const NT x = move(BC, xi.x), y = move(BC, xi.y), z = move(BC, xi.z);
+    xi = mk<NT>(move(NX, xi.x), move(NX, xi.y), move(NX, xi.z));
+    const NT a = (c == 0) ? x : (c == 1) ? y : z, b = (c == 0) ? y : (c == 1) ? z : x, d = (c == 0) ? z : (c == 1) ? x : y;
+    return {(double)a, (double)b, (double)d};
+  };
   // log layout of this lane (logLayerParams, core/junction.hpp:1580-1636):
   // its m channel, if it writes one, and the resistance channels after the
   // m channels of all layers
@@ -767,10 +806,56 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     }
   };
 
+  // Exact sets with few records: whether a record feeds each scalar slot the
+  // set has, as weights of one FMA a slot (the general form finds a record's
+  // slot by a tree of scalar branches, some 30 instructions a step).
+  constexpr bool SLOTW = DYNS && (FM & F_EXACT) != 0 && ND >= 1 && ND <= 2 &&
+                         !(FM & (F_ANIS2 | F_IEC | F_IEC2 | F_IDMI | F_DIPOLE | F_SOT2 | F_DYNH));
+  constexpr int NW = SLOTW ? ND : 1;
+  [[maybe_unused]] double wK[NW], wI[NW], wFL[NW], wDL[NW];
+  if constexpr (SLOTW) {
+#pragma unroll
+    for (int r = 0; r < NW; ++r) {
+      const int slot = (g.dmeta[r] >> 8) & 0xff;
+      wK[r] = slot == CMTJ_SLOT_K ? 1.0 : 0.0;
+      wI[r] = slot == CMTJ_SLOT_CURRENT ? 1.0 : 0.0;
+      wFL[r] = slot == CMTJ_SLOT_FL ? 1.0 : 0.0;
+      wDL[r] = slot == CMTJ_SLOT_DL ? 1.0 : 0.0;
+    }
+  }
+  // Trapezoids of stochastic runs: where every record of the wave stays on one
+  // of its straight pieces over a block, its value there is la + lc (t - lt).
+  constexpr bool LINES = SOLVER == CMTJ_EULER_HEUN && (FM & F_KTRAP) != 0 && ND >= 1;
+  constexpr int NLN = LINES ? ND : 1;
+  [[maybe_unused]] double la[NLN], lc[NLN], lt[NLN];
+  [[maybe_unused]] bool lines = false;
+  auto set_lines = [&](uint32_t a, uint32_t b) __attribute__((always_inline)) {  // steps a to b
+    if constexpr (LINES) {
+      const double ta = (double)a * dt, tb = (double)b * dt;
+      bool ok = true;
+#pragma unroll
+      for (int r = 0; r < NLN; ++r) {
+        const double t1 = dr[r].p1, t2 = t1 + dr[r].p2, t3 = t2 + dr[r].p3, t4 = t1 + 2 * dr[r].p2 + dr[r].p3;
+        auto piece = [&](double t) { return (t < t1) ? 0 : (t <= t2) ? 1 : (t <= t3) ? 2 : (t <= t4) ? 3 : 4; };
+        const int p = piece(ta);
+        ok = ok && p == piece(tb);
+        double slope;
+        __builtin_memcpy(&slope, &dr[r].tidx, sizeof slope);
+        lc[r] = p == 1 ? slope : p == 3 ? -slope : 0.0;
+        lt[r] = p == 1 ? t1 : p == 3 ? t3 : 0.0;
+        la[r] = (p == 2 || p == 3) ? dr[r].A : 0.0;
+      }
+      lines = __ballot(!ok) == 0ull;
+    }
+  };
+
   // Value of record r at the present stage time (ts): sine kinds from their
   // carried phase, the others from the waveform.
   auto rec_value = [&](auto ft_tag, int r, double ts, int stage) __attribute__((always_inline)) -> double {
     constexpr bool FT = decltype(ft_tag)::value;
+    if constexpr (LINES) {
+      if (lines) return fma(lc[r], ts - lt[r], la[r]);
+    }
     if constexpr (!OSC) {
       return wave_value<double, FT, FM>(g.dmeta[r] & 0xff, dr[r], g, ts, i, stage, sps);
     } else {
@@ -883,8 +968,16 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     [[maybe_unused]] const double gH = group_field_cl();
     // ---- drives at ts: this component's field slots and the layer's scalar
     // slots (the slot of a record is wave-uniform: one scalar branch)
-    auto route = [&](CLDrive& d, int meta, bool on, double v) __attribute__((always_inline)) {
+    auto route = [&](CLDrive& d, int r, int meta, bool on, double v) __attribute__((always_inline)) {
       const double x = on ? v : 0.0;
+      if constexpr (SLOTW) {
+        d.K = fma(wK[r], x, d.K);
+        d.I = fma(wI[r], x, d.I);
+        d.FL = fma(wFL[r], x, d.FL);
+        d.DL = fma(wDL[r], x, d.DL);
+        if (t_driven) d.T += ((meta >> 8) & 0xff) == CMTJ_SLOT_TEMPERATURE ? x : 0.0;
+        return;
+      }
       const int slot = (meta >> 8) & 0xff;
       if (!DYNS || slot < CMTJ_SLOT_K) {
         d.H = fma(K.g, x, d.H);
@@ -919,11 +1012,11 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
           if (inwin) {
 #pragma unroll
             for (int r = 0; r < NR; ++r)
-              if (ND >= 0 || r < g.ndyn) route(d, g.dmeta[r], sel[r], rec_value(ft_tag, r, ts, stage));
+              if (ND >= 0 || r < g.ndyn) route(d, r, g.dmeta[r], sel[r], rec_value(ft_tag, r, ts, stage));
             for (int r = DREG; ND < 0 && !(FM & F_EXACT) && r < g.ndyn; ++r) {
               const DynRec rr = load_rec<FM>(g.dyn + (size_t)r * g.n + inst);
               constexpr bool FT = decltype(ft_tag)::value;
-              route(d, g.dmeta[r], feeds_lane(g.dmeta[r]),
+              route(d, r, g.dmeta[r], feeds_lane(g.dmeta[r]),
                     wave_value<double, FT, FM>(g.dmeta[r] & 0xff, rr, g, ts, i, stage, sps));
             }
           }
@@ -1068,23 +1161,25 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     } else if constexpr (F64) {
       // stochasticTorque (core/junction.hpp:824-831) with the layer's three
       // normals of the shared Philox stream: -gamma/(1 + a^2) m x (dW + a m x dW)
+      // dW scaled by -gamma/(1 + a^2) and sqrt(dt), so this is the kick itself
       auto noise = [&](const Rot<double>& s, const Rot<double>& dW) __attribute__((always_inline)) -> double {
-        return cross_a(s, fma(K.alpha, cross_b(s, dW), dW.b), fma(K.alpha, cross_c2(s, dW), dW.c)) * K.gconv;
+        return cross_a(s, fma(K.alpha, cross_b(s, dW), dW.b), fma(K.alpha, cross_c2(s, dW), dW.c));
       };
       const double f0 = torque(m, d0, B0, nb);
       Rot<double> dW{0.0, 0.0, 0.0};
       double g0 = 0.0;
       if (CMTJ_HAS(F_THERMAL)) {
-        const V3<double> xi = thermal_normals<double>(seed, stream, i, (uint32_t)lyr);
-        const double sg = K.therm ? sqrt(K.sig2 * d0.T) : 0.0;
-        dW = {comp(xi, c) * sg, comp(xi, c1) * sg, comp(xi, c2) * sg};
+        const Rot<double> n = next_normals();
+        double sg = K.sg0;
+        if (t_driven) sg = K.therm ? sqrt(K.sig2 * d0.T) * K.kick : 0.0;
+        dW = {n.a * sg, n.b * sg, n.c * sg};
         g0 = noise(m, dW);
       }
       if constexpr (SOLVER == CMTJ_HEUN) {
         // heunSolverStep (core/junction.hpp:1756-1815): a predictor m + f dt
         // + g sqrt(dt), whose neighbours feed the corrector's second
         // evaluation at t + dt; the same dW in both
-        const Rot<double> mN = rot3(m.a + f0 + g0 * sdt);
+        const Rot<double> mN = rot3(m.a + f0 + g0);
         Rot<double> nN[2] = {nb[0], nb[1]};
         neighbours(nN, mN.a);
         turn();
@@ -1092,12 +1187,12 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         const CLDrive d1 = drive(FTT, t + dt, 1);
         const double f1 = torque(mN, d1, frozen(d1, nN), nN);
         mn = m.a + (f0 + f1) * 0.5;
-        if (CMTJ_HAS(F_THERMAL)) mn = mn + ((g0 + noise(mN, dW)) * 0.5) * sdt;
+        if (CMTJ_HAS(F_THERMAL)) mn = fma(0.5, g0 + noise(mN, dW), mn);
       } else {
         // eulerHeunSolverStep (core/junction.hpp:1709-1754): drift at t, the
         // stochastic torque at m and at m + g sqrt(dt), one dW per step
         mn = m.a + f0;
-        if (CMTJ_HAS(F_THERMAL)) mn = mn + ((g0 + noise(rot3(m.a + g0 * sdt), dW)) * 0.5) * sdt;
+        if (CMTJ_HAS(F_THERMAL)) mn = fma(0.5, g0 + noise(rot3(m.a + g0), dW), mn);
         turn();
         turn();
       }
@@ -1153,9 +1248,16 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         mnew = ms;
       }
     } else {
-      // a stochastic step's length is off by the square of its kick
-      const double ss = lact ? e + 1.0 : 0.0;
-      mnew = rot3((ss != 0.0) ? mn / sqrt(ss) : mn);
+      // a stochastic step's length is off by the square of its kick: the
+      // series within its range, the root and division beyond
+      const double p = e * fma(e, fma(e, fma(e, len4, len3), len2), -0.5);
+      mnew = {fma(mn, p, mn), fma(mnew.b, p, mnew.b), fma(mnew.c, p, mnew.c)};
+      const bool near = fabs(e) <= kUnitRange;
+      if (__builtin_expect(__ballot(!near) != 0ull, 0)) {
+        const double ss = lact ? e + 1.0 : 0.0;
+        const Rot<double> ex = rot3((ss != 0.0) ? mn / sqrt(ss) : mn);
+        mnew = {near ? mnew.a : ex.a, near ? mnew.b : ex.b, near ? mnew.c : ex.c};
+      }
     }
     // the reference updates layers in turn and stops at the first NaN
     // layer; layers up to and including it take the new value (RK4 only:
@@ -1266,9 +1368,15 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
             if (u0 != 0u && a == 0u) seek();
           }
           if constexpr (SOLVER != CMTJ_RK4) {
-            for (uint32_t u = u0; u < ue; ++u) {
-              i = i0 + u;
-              step(drv_tag, I0{}, std::false_type{});
+            set_lines(i0 + u0, i0 + ue - 1u);
+            for (uint32_t u = u0; u < ue;) {
+              draw(i0 + u);
+              const uint32_t un = min(u + 4u, ue);
+#pragma nounroll
+              for (; u < un; ++u) {
+                i = i0 + u;
+                step(drv_tag, I0{}, std::false_type{});
+              }
             }
           } else {
             // steps without a per-step NaN test; a block that meets a NaN or

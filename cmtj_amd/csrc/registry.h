@@ -95,6 +95,11 @@ KTable kernels_group_cl();  // Kanao / Nomura groups on one lane per component
    (const void*)&cmtj::k_junction_cl<L, FM, ND, true, CMTJ_EULER_HEUN>,                              \
    "k_junction_cl<double," #L ",EulerHeun," #FM "," #ND ">", (ND) + 1}
 
+// FP32 batches: the same with binary32 normals
+#define CMTJ_KC32S(L, S, FM, ND)                                                                   \
+  {CMTJ_FP32, L, 4 * (L), S, FM, false, (const void*)&cmtj::k_junction_cl<L, FM, ND, true, S, 0, false, 0, true>, \
+   "k_junction_cl<normals f32," #L "," #S "," #FM "," #ND ">", (ND) + 1}
+
 #define CMTJ_KC64H(L, FM, ND)                                                                      \
   {CMTJ_FP64, L, 4 * (L), CMTJ_HEUN, FM, false, (const void*)&cmtj::k_junction_cl<L, FM, ND, true, CMTJ_HEUN>, \
    "k_junction_cl<double," #L ",Heun," #FM "," #ND ">", (ND) + 1}
