@@ -234,16 +234,15 @@ __device__ __forceinline__ T comp(V3<T> v, int c) {
 struct CLConst {
   double g, hb, hb1, hb2;         // the factor; constant field at c, c + 1, c + 2
   double an0, an1, an2;           // anisotropy axis at c, c + 1, c + 2
-  double nm0, nm1, nm2;           // diagonal demagnetisation x Ms / mu0
   Rot<double> A0, A1, A2;         // rows c, c + 1, c + 2 of the field's constant matrix (demagnetisation,
                                   // constant first-order anisotropy) against components c, c + 1, c + 2
   double alpha;
   double jn[2];                   // bilinear IEC towards neighbour n (constant J)
   // binary64 kernels: the layer's scalar drives (constant parts) and spin
   // torques
-  double bK, bK2, bI, bFL, bDL, bT, bFL2, bDL2;
-  double bJ[2], bJ2[2], bD[2];    // IEC, biquadratic IEC, this component of the IDMI vector, per neighbour
-  double n01, n02, n10, n12, n20, n21;  // off-diagonal demag rows c, c + 1, c + 2 against the other components
+  double k2, bI, bFL, bDL, bT, bFL2, bDL2;  // k2: 4 g K2 / Ms
+  double bJ2[2];                  // 2 g J2 / (Ms t) towards neighbour n
+  double Db[2], Dc[2];            // -g / (Ms t) times components c + 1, c + 2 of the IDMI vector of neighbour n
   double dp[2][3];                // dipole tensor rows towards neighbour n
   double ginv_ms, ginv_mst;       // g / Ms, g / (Ms t)
   Rot<double> ref, ref2;          // reference vectors: fixed (for the torque and the classic resistance), secondary
@@ -258,11 +257,16 @@ struct CLConst {
   bool stt, alt, dyn_sot, stat_i, therm;  // STT; its alternative form; SOT from drivers; current-driven torque; thermal
 };
 
-// The drives of one stage time as a binary64 lane sees them: its (scaled)
-// field component, its layer's scalar slots and, per neighbour, the coupling.
+// The drives of one stage time as a lane sees them: its (scaled) field
+// component and its layer's scalar slots.
+struct CLRows {
+  Rot<double> a, b, c;            // rows c, c + 1, c + 2
+};
 struct CLDrive {
-  double H, K, K2, I, FL, DL, T, FL2, DL2;
-  double J[2], J2[2], D[2];
+  double H;                       // with scalar drives: with all that the stage's m does not change
+  double kd, k2;                  // 2 g K / Ms beyond the constant matrix's, 4 g K2 / Ms
+  double I, FL, DL, T, FL2, DL2;
+  double J2[2];                   // 2 g J2 / (Ms t)
 };
 
 // Sine of a drive's phase, carried from stage to stage: s and c are sine and
@@ -450,15 +454,10 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     K.an1 = live ? comp(P.anis, c1) : z;
     K.an2 = live ? comp(P.anis, c2) : z;
     const double gm = K.g * P.ms_mu0;
-    const V3<double> nd = mk<double>(P.N[0], P.N[4], P.N[8]);
-    K.nm0 = live ? comp(nd, c) * gm : z;
-    K.nm1 = live ? comp(nd, c1) * gm : z;
-    K.nm2 = live ? comp(nd, c2) * gm : z;
     K.alpha = P.alpha;
     K.ginv_ms = K.g * P.inv_ms;
     K.ginv_mst = K.g * P.inv_mst;
-    K.bK = base.K;
-    K.bK2 = base.K2;
+    K.k2 = live ? (4.0 * base.K2) * K.ginv_ms : z;
     K.bI = base.I;
     K.bFL = base.FL;
     K.bDL = base.DL;
@@ -468,10 +467,10 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       const bool on = live && has_nb(n), top = nb_top(n);
-      K.bJ[n] = on ? (top ? base.Jt : base.Jb) : z;
-      K.bJ2[n] = on ? (top ? base.J2t : base.J2b) : z;
-      K.bD[n] = on ? comp(top ? base.Dt : base.Db, c) : z;
-      K.jn[n] = K.bJ[n] * K.ginv_mst;
+      K.jn[n] = on ? (top ? base.Jt : base.Jb) * K.ginv_mst : z;
+      K.bJ2[n] = on ? (2.0 * (top ? base.J2t : base.J2b)) * K.ginv_mst : z;
+      K.Db[n] = on ? -K.ginv_mst * comp(top ? base.Dt : base.Db, c1) : z;
+      K.Dc[n] = on ? -K.ginv_mst * comp(top ? base.Dt : base.Db, c2) : z;
       K.dp[n][0] = on ? (top ? CL_ENTRY(P.Nt, cc, cc) : CL_ENTRY(P.Nb, cc, cc)) * gm : z;
       K.dp[n][1] = on ? (top ? CL_ENTRY(P.Nt, cc, c1) : CL_ENTRY(P.Nb, cc, c1)) * gm : z;
       K.dp[n][2] = on ? (top ? CL_ENTRY(P.Nt, cc, c2) : CL_ENTRY(P.Nb, cc, c2)) * gm : z;
@@ -486,12 +485,6 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       K.A1 = row(K.an1, c1);
       K.A2 = row(K.an2, c2);
     }
-    K.n01 = live ? CL_ENTRY(P.N, cc, c1) * gm : z;
-    K.n02 = live ? CL_ENTRY(P.N, cc, c2) * gm : z;
-    K.n10 = live ? CL_ENTRY(P.N, c1, cc) * gm : z;
-    K.n12 = live ? CL_ENTRY(P.N, c1, c2) * gm : z;
-    K.n20 = live ? CL_ENTRY(P.N, c2, cc) * gm : z;
-    K.n21 = live ? CL_ENTRY(P.N, c2, c1) * gm : z;
     const V3<double> r1 = mk<double>(Ly.ref[0], Ly.ref[1], Ly.ref[2]);
     const V3<double> r2 = mk<double>(Ly.ref2[0], Ly.ref2[1], Ly.ref2[2]);
     K.ref = {live ? comp(r1, c) : z, live ? comp(r1, c1) : z, live ? comp(r1, c2) : z};
@@ -538,6 +531,12 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   // eta's denominator is lam2 + 1 on every STT lane of the wave (lambda = 1,
   // the usual spacer): the torque then needs no division
   const bool den_const = (FM & F_STT) != 0 && __ballot(K.stt && (K.alt || K.lam2 != 1.0)) == 0ull;
+  // whether a lane of the wave takes its polariser from a neighbour, and
+  // whether a step reads the neighbours at all (else only a log entry's R
+  // does).  Stochastic solvers only: an RK4 step gains nothing from the branch.
+  constexpr bool RK = SOLVER == CMTJ_RK4;
+  const bool nb_pol = RK || (NN > 0 && (FM & (F_STT | F_SOT)) != 0 && __ballot(K.wp[0] != 0.0 || K.wp[1] != 0.0) != 0ull);
+  const bool nb_step = RK || STK || CMTJ_HAS(F_IEC) || CMTJ_HAS(F_IEC2) || CMTJ_HAS(F_IDMI) || CMTJ_HAS(F_DIPOLE) || nb_pol;
   // the length correction's coefficients, held in registers (as literals they
   // would be moved to one at every step)
   double len2 = 0.375, len3 = -0.3125, len4 = 0.2734375;
@@ -563,8 +562,11 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       return K.dyn_sot;
     if (slot == CMTJ_SLOT_J_TOP || slot == CMTJ_SLOT_J2_TOP) return hasT;
     if (slot == CMTJ_SLOT_J_BOTTOM || slot == CMTJ_SLOT_J2_BOTTOM) return hasB;
-    if (slot >= CMTJ_SLOT_IDMI_TOP && slot < CMTJ_SLOT_IDMI_BOTTOM) return hasT && slot - CMTJ_SLOT_IDMI_TOP == c;
-    if (slot >= CMTJ_SLOT_IDMI_BOTTOM && slot < CMTJ_NSLOT) return hasB && slot - CMTJ_SLOT_IDMI_BOTTOM == c;
+    // (a component of the IDMI vector turns into field components across it)
+    if (slot >= CMTJ_SLOT_IDMI_TOP && slot < CMTJ_SLOT_IDMI_BOTTOM)
+      return hasT && c < 3 && slot - CMTJ_SLOT_IDMI_TOP != c;
+    if (slot >= CMTJ_SLOT_IDMI_BOTTOM && slot < CMTJ_NSLOT)
+      return hasB && c < 3 && slot - CMTJ_SLOT_IDMI_BOTTOM != c;
     return true;
   };
 #pragma unroll
@@ -579,8 +581,11 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         if ((FM & F_KSINE) || sine_kind(g.dmeta[k] & 0xff)) {
           const double w = M_PI * dr[k].p1 * dt;  // half a step's advance
           const double sw = sin(0.5 * w);
-          osc[k].sh = sin(w);
-          osc[k].cm = -2.0 * sw * sw;
+          // a lane the record does not feed carries zeros: what is not finite
+          // stays with the layer it drives
+          osc[k].sh = sel[k] ? sin(w) : 0.0;
+          osc[k].cm = sel[k] ? -2.0 * sw * sw : 0.0;
+          dr[k].A = sel[k] ? dr[k].A : 0.0;
         }
       }
     } else {
@@ -588,14 +593,26 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       sel[k] = false;
     }
   }
-  // whether a drive moves a temperature (else the noise strength is sg0)
-  [[maybe_unused]] bool t_driven = false;
-  if constexpr (DYNS && (FM & F_THERMAL)) {
+  // whether a drive moves a temperature (else the noise strength is sg0), an
+  // anisotropy (else it is in the constant matrix), a biquadratic coupling
+  // (else it joins the matrix once a step), a field term (else one field
+  // serves the stages)
+  [[maybe_unused]] bool t_driven = false, k_driven = false, j2_driven = false, h_driven = false;
+  auto field_slot = [](int slot) {
+    return slot < CMTJ_SLOT_K || slot == CMTJ_SLOT_J_TOP || slot == CMTJ_SLOT_J_BOTTOM || slot >= CMTJ_SLOT_IDMI_TOP;
+  };
+  if constexpr (DYNS) {
+    auto note = [&](int r) {
+      const int slot = (g.dmeta[r] >> 8) & 0xff;
+      t_driven |= slot == CMTJ_SLOT_TEMPERATURE;
+      k_driven |= slot == CMTJ_SLOT_K;
+      j2_driven |= slot == CMTJ_SLOT_J2_TOP || slot == CMTJ_SLOT_J2_BOTTOM;
+      h_driven |= field_slot(slot);
+    };
 #pragma unroll
     for (int k = 0; k < DREG; ++k)
-      if (k < NR && (ND >= 0 || k < g.ndyn)) t_driven |= ((g.dmeta[k] >> 8) & 0xff) == CMTJ_SLOT_TEMPERATURE;
-    for (int r = DREG; ND < 0 && !(FM & F_EXACT) && r < g.ndyn; ++r)
-      t_driven |= ((g.dmeta[r] >> 8) & 0xff) == CMTJ_SLOT_TEMPERATURE;
+      if (k < NR && (ND >= 0 || k < g.ndyn)) note(k);
+    for (int r = DREG; ND < 0 && !(FM & F_EXACT) && r < g.ndyn; ++r) note(r);
   }
   // The layer's normals of four steps at a time: lane c of the quad draws
   // those of step i + c (counter-based, so any lane can), and the step in turn
@@ -817,7 +834,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
 #pragma unroll
     for (int r = 0; r < NW; ++r) {
       const int slot = (g.dmeta[r] >> 8) & 0xff;
-      wK[r] = slot == CMTJ_SLOT_K ? 1.0 : 0.0;
+      wK[r] = slot == CMTJ_SLOT_K ? 2.0 * K.ginv_ms : 0.0;
       wI[r] = slot == CMTJ_SLOT_CURRENT ? 1.0 : 0.0;
       wFL[r] = slot == CMTJ_SLOT_FL ? 1.0 : 0.0;
       wDL[r] = slot == CMTJ_SLOT_DL ? 1.0 : 0.0;
@@ -849,15 +866,16 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     }
   };
 
-  // Value of record r at the present stage time (ts): sine kinds from their
+  // Value of record r at the present stage time (ts), 0 on lanes it does not feed: sine kinds from their
   // carried phase, the others from the waveform.
   auto rec_value = [&](auto ft_tag, int r, double ts, int stage) __attribute__((always_inline)) -> double {
     constexpr bool FT = decltype(ft_tag)::value;
     if constexpr (LINES) {
-      if (lines) return fma(lc[r], ts - lt[r], la[r]);
+      if (lines) return sel[r] ? fma(lc[r], ts - lt[r], la[r]) : 0.0;
     }
     if constexpr (!OSC) {
-      return wave_value<double, FT, FM>(g.dmeta[r] & 0xff, dr[r], g, ts, i, stage, sps);
+      const double v = wave_value<double, FT, FM>(g.dmeta[r] & 0xff, dr[r], g, ts, i, stage, sps);
+      return sel[r] ? v : 0.0;
     } else {
       const int ty = (FM & F_KSINE) ? (int)CMTJ_SINE : (g.dmeta[r] & 0xff);
       if (sine_kind(ty)) {
@@ -865,7 +883,8 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         if (ty == CMTJ_SINE) return v;
         return ty == CMTJ_POSINE ? fabs(v) : ((v <= 0) ? v : 0.0);
       }
-      return wave_value<double, FT, FM>(ty, dr[r], g, ts, i, stage, sps);
+      const double v = wave_value<double, FT, FM>(ty, dr[r], g, ts, i, stage, sps);
+      return sel[r] ? v : 0.0;
     }
   };
   auto turn = [&]() __attribute__((always_inline)) {
@@ -884,8 +903,6 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         if (ND >= 0 || r < g.ndyn) {
           if ((FM & F_KSINE) || sine_kind(g.dmeta[r] & 0xff)) {
             const double2 sc = osc_at(dr[r].p1, dr[r].p2, (double)i0 * dt);
-            // a lane the record does not feed carries zeros: a non-finite
-            // frequency stays with the layer it drives
             osc[r].s = sel[r] ? sc.x : 0.0;
             osc[r].c = sel[r] ? sc.y : 0.0;
           }
@@ -968,10 +985,39 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     [[maybe_unused]] const double gH = group_field_cl();
     // ---- drives at ts: this component's field slots and the layer's scalar
     // slots (the slot of a record is wave-uniform: one scalar branch)
-    auto route = [&](CLDrive& d, int r, int meta, bool on, double v) __attribute__((always_inline)) {
-      const double x = on ? v : 0.0;
+    // With scalar drives, what of the field a stage's m does not change joins
+    // d.H: constant field and couplings once per step (IEC, :654-675; IDMI,
+    // :677-693; dipole tensors, :579-586, with this layer's Ms), and a record
+    // of a field, IEC or IDMI slot by one FMA on its coefficient in this
+    // lane's component, which the frozen neighbours fix for the step.
+    auto base_field = [&](const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> double {
+      double b = K.hb;
+#pragma unroll
+      for (int n = 0; n < NN; ++n) {
+        if (CMTJ_HAS(F_IEC) || CMTJ_HAS(F_IEC2)) b = fma(nbs[n].a, K.jn[n], b);
+        if (CMTJ_HAS(F_IDMI)) b = fma(K.Db[n], nbs[n].c, fma(-K.Dc[n], nbs[n].b, b));
+        if (CMTJ_HAS(F_DIPOLE))
+          b = fma(-K.dp[n][0], nbs[n].a, fma(-K.dp[n][1], nbs[n].b, fma(-K.dp[n][2], nbs[n].c, b)));
+      }
+      return b;
+    };
+    auto coef = [&](int slot, const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> double {
+      if (slot < CMTJ_SLOT_K) return K.g;
+      if constexpr (NN > 0) {
+        const bool low = slot == CMTJ_SLOT_J_BOTTOM || slot >= CMTJ_SLOT_IDMI_BOTTOM;
+        const bool second = NN > 1 && low;
+        const double na = second ? nbs[1].a : nbs[0].a, n1 = second ? nbs[1].b : nbs[0].b,
+                     n2 = second ? nbs[1].c : nbs[0].c;
+        if (slot < CMTJ_SLOT_IDMI_TOP) return K.ginv_mst * na;
+        const int k = slot - (low ? CMTJ_SLOT_IDMI_BOTTOM : CMTJ_SLOT_IDMI_TOP);
+        return K.ginv_mst * (k == c1 ? -n2 : n1);  // -(e_k x n) of component c; lanes of component k are not fed
+      } else {
+        return 0.0;
+      }
+    };
+    auto route = [&](CLDrive& d, int r, int meta, double x, double cf) __attribute__((always_inline)) {
       if constexpr (SLOTW) {
-        d.K = fma(wK[r], x, d.K);
+        d.kd = fma(wK[r], x, d.kd);
         d.I = fma(wI[r], x, d.I);
         d.FL = fma(wFL[r], x, d.FL);
         d.DL = fma(wDL[r], x, d.DL);
@@ -979,31 +1025,29 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         return;
       }
       const int slot = (meta >> 8) & 0xff;
-      if (!DYNS || slot < CMTJ_SLOT_K) {
-        d.H = fma(K.g, x, d.H);
+      if (!DYNS || field_slot(slot)) {
+        d.H = fma(cf, x, d.H);
         return;
       }
       if constexpr (DYNS) {
         switch (slot) {
-          case CMTJ_SLOT_K: d.K += x; break;
-          case CMTJ_SLOT_K2: d.K2 += x; break;
+          case CMTJ_SLOT_K: d.kd = fma(2.0 * K.ginv_ms, x, d.kd); break;
+          case CMTJ_SLOT_K2: d.k2 = fma(4.0 * K.ginv_ms, x, d.k2); break;
           case CMTJ_SLOT_CURRENT: d.I += x; break;
           case CMTJ_SLOT_FL: d.FL += x; break;
           case CMTJ_SLOT_DL: d.DL += x; break;
           case CMTJ_SLOT_FL2: d.FL2 += x; break;
           case CMTJ_SLOT_DL2: d.DL2 += x; break;
           case CMTJ_SLOT_TEMPERATURE: d.T += x; break;
-          case CMTJ_SLOT_J_TOP: d.J[0] += x; break;
-          case CMTJ_SLOT_J_BOTTOM: d.J[L == 2 ? 0 : 1] += x; break;
-          case CMTJ_SLOT_J2_TOP: d.J2[0] += x; break;
-          case CMTJ_SLOT_J2_BOTTOM: d.J2[L == 2 ? 0 : 1] += x; break;
-          default: d.D[(L == 2 || slot < CMTJ_SLOT_IDMI_BOTTOM) ? 0 : 1] += x; break;
+          case CMTJ_SLOT_J2_TOP: d.J2[0] = fma(2.0 * K.ginv_mst, x, d.J2[0]); break;
+          default: d.J2[L == 2 ? 0 : 1] = fma(2.0 * K.ginv_mst, x, d.J2[L == 2 ? 0 : 1]); break;
         }
       }
     };
-    auto drive = [&](auto ft_tag, double ts, int stage) __attribute__((always_inline)) -> CLDrive {
-      CLDrive d{K.hb, K.bK, K.bK2, K.bI, K.bFL, K.bDL, K.bT, K.bFL2, K.bDL2, {K.bJ[0], K.bJ[1]},
-                {K.bJ2[0], K.bJ2[1]}, {K.bD[0], K.bD[1]}};
+    // drives at ts on the field b, the neighbours being nbs
+    auto drive = [&](auto ft_tag, double ts, int stage, double b,
+                     const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> CLDrive {
+      CLDrive d{b, 0.0, K.k2, K.bI, K.bFL, K.bDL, K.bT, K.bFL2, K.bDL2, {K.bJ2[0], K.bJ2[1]}};
       if constexpr (DRIVEN) {
         if (CMTJ_HAS(F_DYNH) || CMTJ_HAS(F_DYN)) {
           bool inwin = true;
@@ -1012,12 +1056,15 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
           if (inwin) {
 #pragma unroll
             for (int r = 0; r < NR; ++r)
-              if (ND >= 0 || r < g.ndyn) route(d, r, g.dmeta[r], sel[r], rec_value(ft_tag, r, ts, stage));
+              if (ND >= 0 || r < g.ndyn)
+                route(d, r, g.dmeta[r], rec_value(ft_tag, r, ts, stage),
+                      DYNS ? coef((g.dmeta[r] >> 8) & 0xff, nbs) : K.g);
             for (int r = DREG; ND < 0 && !(FM & F_EXACT) && r < g.ndyn; ++r) {
               const DynRec rr = load_rec<FM>(g.dyn + (size_t)r * g.n + inst);
               constexpr bool FT = decltype(ft_tag)::value;
-              route(d, r, g.dmeta[r], feeds_lane(g.dmeta[r]),
-                    wave_value<double, FT, FM>(g.dmeta[r] & 0xff, rr, g, ts, i, stage, sps));
+              const double v = wave_value<double, FT, FM>(g.dmeta[r] & 0xff, rr, g, ts, i, stage, sps);
+              route(d, r, g.dmeta[r], feeds_lane(g.dmeta[r]) ? v : 0.0,
+                    DYNS ? coef((g.dmeta[r] >> 8) & 0xff, nbs) : K.g);
             }
           }
         }
@@ -1027,11 +1074,15 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       if constexpr (STK) d.I = K.stat_i ? ((stage == 0) ? sI[0] : (stage == 1) ? sI[1] : sI[2]) : 0.0;
       return d;
     };
-    // ---- what of the field a stage's m does not change: drives and the
-    // frozen neighbours' terms (IEC, :654-675; IDMI, :677-693; dipole
-    // tensors, :579-586, with this layer's Ms)
+    constexpr bool TERMS = DYNS || (FM & (F_IDMI | F_DIPOLE)) != 0;  // base_field in d.H
+    auto start_field = [&](const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> double {
+      double b = TERMS ? base_field(nbs) : K.hb;
+      if constexpr (GW > 0) b += gH;
+      return b;
+    };
+    // ---- what of the field a stage's m does not change, all components
     auto frozen = [&](const CLDrive& d, const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> Rot<double> {
-      if constexpr (!DRIVEN && !DYNS && !(FM & (F_IDMI | F_DIPOLE)) && GW == 0) {
+      if constexpr ((SLOTW || (!DRIVEN && !TERMS)) && GW == 0) {
         // constant field and coupling: the neighbours' components are in the lane
         Rot<double> B{K.hb, K.hb1, K.hb2};
         if (CMTJ_HAS(F_IEC)) {
@@ -1041,50 +1092,47 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         }
         return B;
       }
-      double b = (GW > 0) ? d.H + gH : d.H;
+      double b = d.H;
+      if constexpr (!TERMS) {
 #pragma unroll
-      for (int n = 0; n < NN; ++n) {
-        if (CMTJ_HAS(F_IEC) || CMTJ_HAS(F_IEC2)) b = fma(nbs[n].a, DYNS ? d.J[n] * K.ginv_mst : K.jn[n], b);
-        if (CMTJ_HAS(F_IDMI)) {
-          const Rot<double> D = rot3(d.D[n]);
-          b = fma(-K.ginv_mst, cross_a(D, nbs[n].b, nbs[n].c), b);
-        }
-        if (CMTJ_HAS(F_DIPOLE))
-          b = fma(-K.dp[n][0], nbs[n].a, fma(-K.dp[n][1], nbs[n].b, fma(-K.dp[n][2], nbs[n].c, b)));
+        for (int n = 0; n < NN; ++n)
+          if (CMTJ_HAS(F_IEC)) b = fma(nbs[n].a, K.jn[n], b);
       }
       return rot3(b);
+    };
+    // ---- the field's matrix: the constant one, with the biquadratic
+    // coupling's rank-one terms 2 J2 (nb . s) nb / (Ms t) of the frozen
+    // neighbours
+    auto matrix = [&](const CLDrive& d, const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> CLRows {
+      CLRows A{K.A0, K.A1, K.A2};
+      if (CMTJ_HAS(F_IEC2)) {
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+          const double w = d.J2[n];
+          const Rot<double> v = nbs[n];
+          const double wa = w * v.a, wb = w * v.b, wc = w * v.c;
+          A.a = {fma(wa, v.a, A.a.a), fma(wa, v.b, A.a.b), fma(wa, v.c, A.a.c)};
+          A.b = {fma(wb, v.a, A.b.a), fma(wb, v.b, A.b.b), fma(wb, v.c, A.b.c)};
+          A.c = {fma(wc, v.a, A.c.a), fma(wc, v.b, A.c.b), fma(wc, v.c, A.c.c)};
+        }
+      }
+      return A;
     };
     // ---- field at m = s (all three components; calculateHeffDipoleInjection,
     // core/junction.hpp:590-622), scaled by K.g
     auto field = [&](const Rot<double>& s, const CLDrive& d, const Rot<double>& B,
-                     const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> Rot<double> {
-      auto along = [&](const Rot<double>& A, double x) {
-        return fma(A.c, s.c, fma(A.b, s.b, fma(A.a, s.a, x)));
+                     const CLRows& A) __attribute__((always_inline)) -> Rot<double> {
+      auto along = [&](const Rot<double>& r, double x) {
+        return fma(r.c, s.c, fma(r.b, s.b, fma(r.a, s.a, x)));
       };
-      Rot<double> h;
-      if constexpr (!(FM & (F_DYN | F_ANIS2))) {
-        h = {along(K.A0, B.a), along(K.A1, B.b), along(K.A2, B.c)};
-      } else {
-        h = {fma(-K.nm0, s.a, B.a), fma(-K.nm1, s.b, B.b), fma(-K.nm2, s.c, B.c)};
-        if (CMTJ_HAS(F_ANIS) || CMTJ_HAS(F_ANIS2)) {
+      Rot<double> h{along(A.a, B.a), along(A.b, B.b), along(A.c, B.c)};
+      if constexpr ((FM & (F_DYN | F_ANIS2)) != 0) {
+        if (CMTJ_HAS(F_ANIS2) || k_driven) {
+          // calculateSecondOrderAnisotropy (:645-652): 4 K2 (anis . m)^3 / Ms,
+          // and what drives add to the first order
           const double u = fma(K.an2, s.c, fma(K.an1, s.b, K.an0 * s.a));  // anis . m
-          // calculateSecondOrderAnisotropy (:645-652): 4 K2 (anis . m)^3 / Ms
-          double w = (2.0 * d.K) * K.ginv_ms;
-          if (CMTJ_HAS(F_ANIS2)) w = fma((4.0 * d.K2) * K.ginv_ms, u * u, w);
-          w = w * u;
+          const double w = fma(d.k2, u * u, d.kd) * u;
           h = {fma(K.an0, w, h.a), fma(K.an1, w, h.b), fma(K.an2, w, h.c)};
-        }
-        if (CMTJ_HAS(F_DEMAG_OFF)) {
-          h.a = fma(-K.n01, s.b, fma(-K.n02, s.c, h.a));
-          h.b = fma(-K.n10, s.a, fma(-K.n12, s.c, h.b));
-          h.c = fma(-K.n20, s.a, fma(-K.n21, s.b, h.c));
-        }
-      }
-      if (CMTJ_HAS(F_IEC2)) {
-#pragma unroll
-        for (int n = 0; n < NN; ++n) {
-          const double w = ((2.0 * d.J2[n]) * K.ginv_mst) * rdot(nbs[n], s);
-          h = {fma(nbs[n].a, w, h.a), fma(nbs[n].b, w, h.b), fma(nbs[n].c, w, h.c)};
         }
       }
       return h;
@@ -1092,18 +1140,20 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     // ---- dm of a step at m = s (solveLLG, :716-815): m x (h + alpha m x h
     // + sum of a p + b m x p over the spin torques' polarisers p).  As cross
     // products throughout: the initial m of a run need not have unit length.
-    auto torque = [&](const Rot<double>& s, const CLDrive& d, const Rot<double>& B,
+    auto torque = [&](const Rot<double>& s, const CLDrive& d, const Rot<double>& B, const CLRows& A,
                       const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> double {
-      const Rot<double> h = field(s, d, B, nbs);
+      const Rot<double> h = field(s, d, B, A);
       double wb = fma(K.alpha, cross_b(s, h), h.b), wc = fma(K.alpha, cross_c2(s, h), h.c);
       if constexpr ((FM & (F_STT | F_SOT)) != 0) {
         if (CMTJ_HAS(F_STT) || CMTJ_HAS(F_SOT)) {
           // the layer's reference vector: fixed, or the start-of-step top /
           // bottom neighbour
           Rot<double> p = K.pol;
+          if (nb_pol) {
 #pragma unroll
-          for (int n = 0; n < NN; ++n)
-            p = {fma(K.wp[n], nbs[n].a, p.a), fma(K.wp[n], nbs[n].b, p.b), fma(K.wp[n], nbs[n].c, p.c)};
+            for (int n = 0; n < NN; ++n)
+              p = {fma(K.wp[n], nbs[n].a, p.a), fma(K.wp[n], nbs[n].b, p.b), fma(K.wp[n], nbs[n].c, p.c)};
+          }
           double a = 0.0, b = 0.0;
           if (CMTJ_HAS(F_STT)) {
             // Slonczewski STT (:743-769)
@@ -1137,26 +1187,29 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       return cross_a(s, wb, wc);
     };
     constexpr std::integral_constant<bool, !F64> FTT{};  // binary32 path: single-precision transcendentals
-    const CLDrive d0 = drive(FTT, t, 0);
+    const double b0 = start_field(nb);
+    const CLDrive d0 = drive(FTT, t, 0, b0, nb);
     const Rot<double> B0 = frozen(d0, nb);
+    const CLRows M0 = matrix(d0, nb);
     if constexpr (F64 && SOLVER == CMTJ_RK4) {
       // rk4_step (core/junction.hpp:1017-1041) in binary64
-      const double k1 = torque(m, d0, B0, nb);
+      const double k1 = torque(m, d0, B0, M0, nb);
       CLDrive d1 = d0;
       Rot<double> B1 = B0;
-      if constexpr (DRIVEN || STK) {
-        turn();
-        d1 = drive(FTT, t + 0.5 * dt, 1);
-        if constexpr (DRIVEN) B1 = frozen(d1, nb);
-      }
-      const double k2 = torque(rot3(fma(0.5, k1, m.a)), d1, B1, nb);
-      const double k3 = torque(rot3(fma(0.5, k2, m.a)), d1, B1, nb);
-      if constexpr (DRIVEN || STK) {
-        turn();
-        d1 = drive(FTT, t + dt, 2);
-        if constexpr (DRIVEN) B1 = frozen(d1, nb);
-      }
-      const double k4 = torque(rot3(m.a + k3), d1, B1, nb);
+      CLRows M1 = M0;
+      auto stage_drives = [&](double ts, int stage) __attribute__((always_inline)) {
+        if constexpr (DRIVEN || STK) {
+          turn();
+          d1 = drive(FTT, ts, stage, b0, nb);
+          if (DRIVEN && (!DYNS || h_driven)) B1 = frozen(d1, nb);
+          if (DYNS && j2_driven) M1 = matrix(d1, nb);
+        }
+      };
+      stage_drives(t + 0.5 * dt, 1);
+      const double k2 = torque(rot3(fma(0.5, k1, m.a)), d1, B1, M1, nb);
+      const double k3 = torque(rot3(fma(0.5, k2, m.a)), d1, B1, M1, nb);
+      stage_drives(t + dt, 2);
+      const double k4 = torque(rot3(m.a + k3), d1, B1, M1, nb);
       mn = fma(fma(2.0, k2 + k3, k1 + k4), 1.0 / 6.0, m.a);
     } else if constexpr (F64) {
       // stochasticTorque (core/junction.hpp:824-831) with the layer's three
@@ -1165,13 +1218,17 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       auto noise = [&](const Rot<double>& s, const Rot<double>& dW) __attribute__((always_inline)) -> double {
         return cross_a(s, fma(K.alpha, cross_b(s, dW), dW.b), fma(K.alpha, cross_c2(s, dW), dW.c));
       };
-      const double f0 = torque(m, d0, B0, nb);
+      const double f0 = torque(m, d0, B0, M0, nb);
       Rot<double> dW{0.0, 0.0, 0.0};
       double g0 = 0.0;
       if (CMTJ_HAS(F_THERMAL)) {
         const Rot<double> n = next_normals();
         double sg = K.sg0;
-        if (t_driven) sg = K.therm ? sqrt(K.sig2 * d0.T) * K.kick : 0.0;
+        if (t_driven) {
+          double T = d0.T;
+          asm volatile("" : "+v"(T));  // (a root taken only here: the compiler would take it at every step)
+          sg = K.therm ? sqrt(K.sig2 * T) * K.kick : 0.0;
+        }
         dW = {n.a * sg, n.b * sg, n.c * sg};
         g0 = noise(m, dW);
       }
@@ -1184,8 +1241,8 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         neighbours(nN, mN.a);
         turn();
         turn();
-        const CLDrive d1 = drive(FTT, t + dt, 1);
-        const double f1 = torque(mN, d1, frozen(d1, nN), nN);
+        const CLDrive d1 = drive(FTT, t + dt, 1, start_field(nN), nN);
+        const double f1 = torque(mN, d1, frozen(d1, nN), matrix(d1, nN), nN);
         mn = m.a + (f0 + f1) * 0.5;
         if (CMTJ_HAS(F_THERMAL)) mn = fma(0.5, g0 + noise(mN, dW), mn);
       } else {
@@ -1198,7 +1255,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       }
     } else {
       // ---- anchor: dm/dt at (m, t) in binary64
-      const Rot<double> h = field(m, d0, B0, nb);
+      const Rot<double> h = field(m, d0, B0, M0);
       const double gb = fma(K.alpha, cross_b(m, h), h.b), gc = fma(K.alpha, cross_c2(m, h), h.c);
       const double k1 = cross_a(m, gb, gc);
       // ---- stages 2-4: binary32 increments about the anchor
@@ -1207,9 +1264,9 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       if constexpr (DRIVEN) {
         // scaled drive increments against the start of the step
         turn();
-        dmid = (float)(drive(FTT, t + 0.5 * dt, 1).H - d0.H);
+        dmid = (float)(drive(FTT, t + 0.5 * dt, 1, b0, nb).H - d0.H);
         turn();
-        dend = (float)(drive(FTT, t + dt, 2).H - d0.H);
+        dend = (float)(drive(FTT, t + dt, 2, b0, nb).H - d0.H);
       }
       mn = m.a + fma((double)stage_increments(KF, (float)k1, m, h, gb, gc, dmid, dend), 1.0 / 6.0, k1);
     }
@@ -1282,10 +1339,12 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     }
     // a step that goes on: new m, neighbours, log entry
     m = mnew;
-    neighbours(nb, m.a);
+    if (nb_step) neighbours(nb, m.a);
     if constexpr (LOGM == 3) {
+      if (!nb_step) neighbours(nb, m.a);
       lv = lane_value();
     } else if (LOGM == 1 || (LOGM == 0 && (uint64_t)i == next_log)) {
+      if (!nb_step) neighbours(nb, m.a);
       const double v = lane_value();
       if (wlog) log_put(f32log, pk, v);
       if (LOGF == 0 && strip) {
