@@ -43,6 +43,7 @@ constexpr int QP_NEXT = 0x39;   // quad_perm [1,2,3,0]: the quad's values move d
 constexpr int DPP_ROW_SHR4 = 0x114;  // lane i reads lane i - 4 (0 outside the row)
 constexpr int DPP_ROW_SHL4 = 0x104;  // lane i reads lane i + 4
 constexpr int DPP_HALF_MIRROR = 0x141;  // lane i reads lane 7 - i of its 8
+constexpr int DPP_MIRROR = 0x140;       // lane i reads lane 15 - i of its row
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -296,6 +297,22 @@ __device__ __forceinline__ bool sine_kind(int type) {
   return type == CMTJ_SINE || type == CMTJ_POSINE || type == CMTJ_HALFSINE;
 }
 
+// Sum over two 16-lane rows of each half wave (ROWS 16), or over the halves
+// (ROWS 32), of a value that is the same in all lanes of a row (half).
+template <int ROWS>
+__device__ __forceinline__ double add_rows(double v) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)u, hi = (unsigned)(u >> 32);
+  // swapped against itself: the first result holds the even row's value in
+  // both rows of a pair, the second the odd row's
+  const auto l = (ROWS == 16) ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false)
+                              : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto h = (ROWS == 16) ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false)
+                              : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0])) +
+         __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
+}
+
 // What the waves of a dipole-coupled group share: the elements' top-layer m
 // scaled by their source strengths, in two copies taken in turn (one barrier
 // a step: a wave writes a copy again only after the barrier of the step
@@ -371,7 +388,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   uint32_t inst;
   int q;
   [[maybe_unused]] const cmtj_stack* sk = nullptr;
-  [[maybe_unused]] int s_j = 0, s_n = 0, s_base = 0, s_lane0 = 0;
+  [[maybe_unused]] int s_j = 0, s_n = 0, s_base = 0;
   [[maybe_unused]] const cmtj_group* gp = nullptr;
   [[maybe_unused]] int g_n = 0, g_e = 0, g_top = 0;
   bool own = true;  // the lanes hold an instance
@@ -387,18 +404,19 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     q = (int)(threadIdx.x % LPI);
     g_top = own ? gp->top[g_e] : 0;
   } else if constexpr (STK) {
-    // lanes of a stack past its members leave at once; a stack never
-    // straddles a wave (pad is a power of two of at most 64)
+    // a stack never straddles a wave (pad is a power of two of at most 64);
+    // lanes past its members stay for the lane moves, as a member without
+    // layers (m = 0)
     const uint32_t pad = g.stack_pad, sid = gl / pad;
     if (sid >= g.stack_n) return;
     sk = g.stack + sid;
     s_n = sk->n_junctions;
     s_j = (int)((gl % pad) / LPI);
-    if (s_j >= s_n) return;
+    own = s_j < s_n;
+    s_j = own ? s_j : 0;
     q = (int)(gl % LPI);
     inst = sid * (uint32_t)s_n + (uint32_t)s_j;
     s_base = (int)(threadIdx.x & ~(pad - 1));
-    s_lane0 = s_base + s_j * LPI;
   } else {
     inst = gl / LPI;
     if (inst >= g.n) return;
@@ -712,6 +730,8 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   [[maybe_unused]] int s_ti = 0;
   [[maybe_unused]] double sI[3] = {0.0, 0.0, 0.0};
   [[maybe_unused]] double sIlog = 0.0, sClog = 0.0;
+  [[maybe_unused]] double s_w = 0.0;
+  [[maybe_unused]] bool s_kcl = false, s_const = false;  // of the whole wave
   [[maybe_unused]] unsigned long long s_mask = 0ull;  // the stack's lanes
   [[maybe_unused]] Rot<double> s_pol = {0.0, 0.0, 0.0};
   if constexpr (STK) {
@@ -720,6 +740,12 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     s_mask = ((g.stack_pad >= 64) ? ~0ull : ((1ull << g.stack_pad) - 1)) << (unsigned)s_base;
     const V3<double> pv = mk<double>(sl.pol[0], sl.pol[1], sl.pol[2]);
     s_pol = {comp(pv, c), comp(pv, c1), comp(pv, c2)};
+    // KCL: the stack's current is I0 (1 + sum_j C_j), C_j = c_j (d_j +- d_{j+1});
+    // taken by members, d_j times c_j +- c_{j-1}, no member needs another's d
+    const double cp = (own && s_j > 0) ? sk->coupling[s_j - 1] : 0.0;
+    s_w = own ? (sl.series ? sl.cj + cp : sl.cj - cp) : 0.0;
+    s_kcl = __ballot(!sl.kcl) == 0ull;
+    s_const = __ballot(sl.current.type != CMTJ_CONSTANT) == 0ull;
   }
 
   // Groups: field of the other elements on this lane's component of its
@@ -980,7 +1006,26 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         const double below = dpp_d<DPP_ROW_SHR4>(dq), above = dpp_d<DPP_ROW_SHL4>(dq);
         dq = (ly == s_ti) ? dq : (ly == s_ti + 1) ? below : above;
       }
-      stack_current(sl, s_j, s_n, s_base, LPI, dq, t, dt, g.tables, i, sI, sIlog, sClog);
+      if (s_kcl) {
+        const double I0 = s_const ? sl.current.constant
+                          : (sl.current.type == CMTJ_TABLE) ? g.tables[(size_t)sl.current.table_index + i]
+                                                            : driver_value(sl.current, t);
+        // sum over the members: every lane of a member's quads holds its term
+        double S = s_w * dpp_d<QP_BC0>(dq);
+        if (L == 1 && g.stack_pad >= 8) S += dpp_d<DPP_HALF_MIRROR>(S);
+        if (g.stack_pad >= 16) S += dpp_d<DPP_MIRROR>(S);
+        if (g.stack_pad >= 32) S = add_rows<16>(S);
+        if (g.stack_pad >= 64) S = add_rows<32>(S);
+        sI[0] = sI[1] = sI[2] = sIlog = fma(I0, S, I0);
+        // C_j of the stack's log, where the step writes an entry
+        if (LOGM == 1 || LOGM == 3 || (LOGM == 0 && (uint64_t)i == next_log)) {
+          const bool last = s_j + 1 >= s_n;
+          const double dn = __shfl(dq, s_base + (last ? s_j : s_j + 1) * LPI, 64);
+          sClog = last ? 0.0 : sl.cj * (sl.series ? dq + dn : dq - dn);
+        }
+      } else {
+        stack_current(sl, s_j, s_n, s_base, LPI, dq, t, dt, g.tables, i, sI, sIlog, sClog);
+      }
     }
     [[maybe_unused]] const double gH = group_field_cl();
     // ---- drives at ts: this component's field slots and the layer's scalar
@@ -1367,7 +1412,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         }
       }
       if constexpr (STK) {
-        if (logging && q == 0) {  // the member's stack channels follow its junction channels
+        if (logging && own && q == 0) {  // the member's stack channels follow its junction channels
           const uint64_t nch = (uint64_t)log_channels(nl, g.mr_mode, g.log_mask);
           log_put(f32log, pk - om + nch * cs, sIlog);
           log_put(f32log, pk - om + (nch + 1) * cs, sClog);
@@ -1592,7 +1637,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   }
   if (S) {
     if (live) S->m[ly][c] = m.a;
-    if (q == 0) {
+    if (own && q == 0) {
       S->step = i;
       S->entries = k;
       S->code = code;
