@@ -260,6 +260,9 @@ struct CLConst {
 
 // The drives of one stage time as a lane sees them: its (scaled) field
 // component and its layer's scalar slots.
+struct CLSpin {
+  Rot<double> B, Q;               // the field with a p, and (b - alpha a) p
+};
 struct CLRows {
   Rot<double> a, b, c;            // rows c, c + 1, c + 2
 };
@@ -555,6 +558,25 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   constexpr bool RK = SOLVER == CMTJ_RK4;
   const bool nb_pol = RK || (NN > 0 && (FM & (F_STT | F_SOT)) != 0 && __ballot(K.wp[0] != 0.0 || K.wp[1] != 0.0) != 0ull);
   const bool nb_step = RK || STK || CMTJ_HAS(F_IEC) || CMTJ_HAS(F_IEC2) || CMTJ_HAS(F_IDMI) || CMTJ_HAS(F_DIPOLE) || nb_pol;
+  // spin torques under constant currents: a p and (b - alpha a) p of a fixed
+  // polariser are constants, of a neighbour two factors (see spin below)
+  constexpr bool SPC = (FM & (F_STT | F_SOT)) != 0 && !DYNS && !STK;
+  static_assert(!SPC || !(FM & F_SOT), "constant currents: STT");
+  [[maybe_unused]] Rot<double> Q0 = {0.0, 0.0, 0.0};
+  [[maybe_unused]] double swa[2] = {0.0, 0.0}, swb[2] = {0.0, 0.0};
+  if constexpr (SPC) {
+    const double w = den_const ? K.bI * K.wc : 0.0;
+    const double a = K.sta * w, b = fma(-K.alpha, a, K.stb * w);
+    K.hb = fma(a, K.pol.a, K.hb);
+    K.hb1 = fma(a, K.pol.b, K.hb1);
+    K.hb2 = fma(a, K.pol.c, K.hb2);
+    Q0 = {b * K.pol.a, b * K.pol.b, b * K.pol.c};
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      swa[n] = a * K.wp[n];
+      swb[n] = b * K.wp[n];
+    }
+  }
   // the length correction's coefficients, held in registers (as literals they
   // would be moved to one at every step)
   double len2 = 0.375, len3 = -0.3125, len4 = 0.2734375;
@@ -1182,35 +1204,42 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       }
       return h;
     };
-    // ---- dm of a step at m = s (solveLLG, :716-815): m x (h + alpha m x h
-    // + sum of a p + b m x p over the spin torques' polarisers p).  As cross
-    // products throughout: the initial m of a run need not have unit length.
-    auto torque = [&](const Rot<double>& s, const CLDrive& d, const Rot<double>& B, const CLRows& A,
-                      const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> double {
-      const Rot<double> h = field(s, d, B, A);
-      double wb = fma(K.alpha, cross_b(s, h), h.b), wc = fma(K.alpha, cross_c2(s, h), h.c);
-      if constexpr ((FM & (F_STT | F_SOT)) != 0) {
-        if (CMTJ_HAS(F_STT) || CMTJ_HAS(F_SOT)) {
-          // the layer's reference vector: fixed, or the start-of-step top /
-          // bottom neighbour
-          Rot<double> p = K.pol;
-          if (nb_pol) {
+    // ---- the spin torques of a stage time (:743-812): a p + b m x p over the
+    // polarisers p, with a, b and p fixed for the stage, joins the field as
+    // a p and the damping's alpha h as (b - alpha a) p, so that a torque costs
+    // what it costs without them and one more (before: eight more; a step of a
+    // spin-torque oscillator 161 -> 128 VALU instructions)
+    auto polariser = [&](const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> Rot<double> {
+      // the layer's reference vector: fixed, or the start-of-step top /
+      // bottom neighbour
+      Rot<double> p = K.pol;
+      if (nb_pol) {
 #pragma unroll
-            for (int n = 0; n < NN; ++n)
-              p = {fma(K.wp[n], nbs[n].a, p.a), fma(K.wp[n], nbs[n].b, p.b), fma(K.wp[n], nbs[n].c, p.c)};
-          }
+        for (int n = 0; n < NN; ++n)
+          p = {fma(K.wp[n], nbs[n].a, p.a), fma(K.wp[n], nbs[n].b, p.b), fma(K.wp[n], nbs[n].c, p.c)};
+      }
+      return p;
+    };
+    const bool spin_on = CMTJ_HAS(F_STT) || CMTJ_HAS(F_SOT);
+    auto spin = [&](const CLDrive& d, const Rot<double> (&nbs)[2], const Rot<double>& B) __attribute__((always_inline)) -> CLSpin {
+      CLSpin r{B, {0.0, 0.0, 0.0}};
+      if constexpr (SPC) {
+        r.Q = Q0;
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+          r.B = {fma(swa[n], nbs[n].a, r.B.a), fma(swa[n], nbs[n].b, r.B.b), fma(swa[n], nbs[n].c, r.B.c)};
+          r.Q = {fma(swb[n], nbs[n].a, r.Q.a), fma(swb[n], nbs[n].b, r.Q.b), fma(swb[n], nbs[n].c, r.Q.c)};
+        }
+      } else if constexpr ((FM & (F_STT | F_SOT)) != 0) {
+        if (spin_on) {
+          const Rot<double> p = polariser(nbs);
           double a = 0.0, b = 0.0;
           if (CMTJ_HAS(F_STT)) {
-            // Slonczewski STT (:743-769)
-            a = K.sta * (d.I * K.wc);
-            b = K.stb * (d.I * K.wc);
-            if (__builtin_expect(!den_const, 0)) {
-              const double mp = rdot(s, p);
-              const double den = K.alt ? fma(K.lam, mp, 1.0) : fma(K.lam2 - 1.0, mp, K.lam2 + 1.0);
-              const double w = d.I * (K.num / den);
-              a = K.stt ? K.sta * w : 0.0;
-              b = K.stt ? K.stb * w : 0.0;
-            }
+            // Slonczewski STT (:743-769) where eta is constant (else torque()
+            // adds it)
+            const double w = den_const ? d.I * K.wc : 0.0;
+            a = K.sta * w;
+            b = K.stb * w;
           }
           if (CMTJ_HAS(F_SOT)) {
             // SOT (:770-812): coefficients from the drivers, or static ones
@@ -1219,42 +1248,73 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
             a = fma(K.ga, Hfl, fma(-K.gaa, Hdl, a));
             b = fma(K.ga, Hdl, fma(K.gaa, Hfl, b));
           }
-          wb = fma(b, cross_b(s, p), fma(a, p.b, wb));
-          wc = fma(b, cross_c2(s, p), fma(a, p.c, wc));
+          const double w = fma(-K.alpha, a, b);
+          r.B = {fma(a, p.a, B.a), fma(a, p.b, B.b), fma(a, p.c, B.c)};
+          r.Q = {w * p.a, w * p.b, w * p.c};
           if (CMTJ_HAS(F_SOT2)) {
             // the secondary reference (dynamic SOT drivers only)
             const double a2 = fma(K.g2, d.FL2, -K.g2a * d.DL2), b2 = fma(K.g2, d.DL2, K.g2a * d.FL2);
-            wb = fma(b2, cross_b(s, K.ref2), fma(a2, K.ref2.b, wb));
-            wc = fma(b2, cross_c2(s, K.ref2), fma(a2, K.ref2.c, wc));
+            const double w2 = fma(-K.alpha, a2, b2);
+            const Rot<double> p2 = K.ref2;
+            r.B = {fma(a2, p2.a, r.B.a), fma(a2, p2.b, r.B.b), fma(a2, p2.c, r.B.c)};
+            r.Q = {fma(w2, p2.a, r.Q.a), fma(w2, p2.b, r.Q.b), fma(w2, p2.c, r.Q.c)};
           }
         }
       }
-      return cross_a(s, wb, wc);
+      return r;
+    };
+    // ---- dm of a step at m = s (solveLLG, :716-815): m x (h + m x (alpha h)),
+    // the spin torques in both.  As cross products throughout: the initial m
+    // of a run need not have unit length.
+    auto torque = [&](const Rot<double>& s, const CLDrive& d, const CLSpin& sp, const CLRows& A,
+                      const Rot<double> (&nbs)[2]) __attribute__((always_inline)) -> double {
+      Rot<double> h = field(s, d, sp.B, A);
+      if constexpr ((FM & (F_STT | F_SOT)) != 0) {
+        if (spin_on) {
+          Rot<double> v{fma(K.alpha, h.a, sp.Q.a), fma(K.alpha, h.b, sp.Q.b), fma(K.alpha, h.c, sp.Q.c)};
+          if (CMTJ_HAS(F_STT) && __builtin_expect(!den_const, 0)) {
+            const Rot<double> p = polariser(nbs);
+            const double mp = rdot(s, p);
+            const double den = K.alt ? fma(K.lam, mp, 1.0) : fma(K.lam2 - 1.0, mp, K.lam2 + 1.0);
+            const double w = d.I * (K.num / den);
+            const double a = K.stt ? K.sta * w : 0.0, b = K.stt ? K.stb * w : 0.0;
+            h = {fma(a, p.a, h.a), fma(a, p.b, h.b), fma(a, p.c, h.c)};
+            v = {fma(b, p.a, v.a), fma(b, p.b, v.b), fma(b, p.c, v.c)};
+          }
+          return cross_a(s, fma(s.c, v.a, fma(-s.a, v.c, h.b)), fma(s.a, v.b, fma(-s.b, v.a, h.c)));
+        }
+      }
+      return cross_a(s, fma(K.alpha, cross_b(s, h), h.b), fma(K.alpha, cross_c2(s, h), h.c));
     };
     constexpr std::integral_constant<bool, !F64> FTT{};  // binary32 path: single-precision transcendentals
     const double b0 = start_field(nb);
     const CLDrive d0 = drive(FTT, t, 0, b0, nb);
     const Rot<double> B0 = frozen(d0, nb);
     const CLRows M0 = matrix(d0, nb);
+    const CLSpin S0 = spin(d0, nb, B0);
     if constexpr (F64 && SOLVER == CMTJ_RK4) {
       // rk4_step (core/junction.hpp:1017-1041) in binary64
-      const double k1 = torque(m, d0, B0, M0, nb);
+      const double k1 = torque(m, d0, S0, M0, nb);
       CLDrive d1 = d0;
       Rot<double> B1 = B0;
       CLRows M1 = M0;
+      CLSpin S1 = S0;
       auto stage_drives = [&](double ts, int stage) __attribute__((always_inline)) {
         if constexpr (DRIVEN || STK) {
+          // (a KCL stack's current is the same at every stage time)
+          if (STK && !DRIVEN && s_kcl) return;
           turn();
           d1 = drive(FTT, ts, stage, b0, nb);
           if (DRIVEN && (!DYNS || h_driven)) B1 = frozen(d1, nb);
           if (DYNS && j2_driven) M1 = matrix(d1, nb);
+          S1 = spin(d1, nb, B1);
         }
       };
       stage_drives(t + 0.5 * dt, 1);
-      const double k2 = torque(rot3(fma(0.5, k1, m.a)), d1, B1, M1, nb);
-      const double k3 = torque(rot3(fma(0.5, k2, m.a)), d1, B1, M1, nb);
+      const double k2 = torque(rot3(fma(0.5, k1, m.a)), d1, S1, M1, nb);
+      const double k3 = torque(rot3(fma(0.5, k2, m.a)), d1, S1, M1, nb);
       stage_drives(t + dt, 2);
-      const double k4 = torque(rot3(m.a + k3), d1, B1, M1, nb);
+      const double k4 = torque(rot3(m.a + k3), d1, S1, M1, nb);
       mn = fma(fma(2.0, k2 + k3, k1 + k4), 1.0 / 6.0, m.a);
     } else if constexpr (F64) {
       // stochasticTorque (core/junction.hpp:824-831) with the layer's three
@@ -1263,7 +1323,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       auto noise = [&](const Rot<double>& s, const Rot<double>& dW) __attribute__((always_inline)) -> double {
         return cross_a(s, fma(K.alpha, cross_b(s, dW), dW.b), fma(K.alpha, cross_c2(s, dW), dW.c));
       };
-      const double f0 = torque(m, d0, B0, M0, nb);
+      const double f0 = torque(m, d0, S0, M0, nb);
       Rot<double> dW{0.0, 0.0, 0.0};
       double g0 = 0.0;
       if (CMTJ_HAS(F_THERMAL)) {
@@ -1287,7 +1347,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         turn();
         turn();
         const CLDrive d1 = drive(FTT, t + dt, 1, start_field(nN), nN);
-        const double f1 = torque(mN, d1, frozen(d1, nN), matrix(d1, nN), nN);
+        const double f1 = torque(mN, d1, spin(d1, nN, frozen(d1, nN)), matrix(d1, nN), nN);
         mn = m.a + (f0 + f1) * 0.5;
         if (CMTJ_HAS(F_THERMAL)) mn = fma(0.5, g0 + noise(mN, dW), mn);
       } else {
