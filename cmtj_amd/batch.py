@@ -373,7 +373,9 @@ class JunctionBatch:
     def fp64_groups(self) -> int:
         """Structure groups of an FP32 batch that run binary64 kernels (spin
         torques or scalar drives on one lane per component, where no
-        binary32 kernel covers them): their arithmetic is the drop-in's."""
+        binary32 kernel covers them): their arithmetic is the drop-in's.
+        (The layer-lane RK4 set of anisotropy, coupling and field steps has
+        binary64 steps in both modes and is not counted.)"""
         return int(self.plan().info.fp64_groups)
 
     def capture(self, device="cuda") -> "JunctionBatch":

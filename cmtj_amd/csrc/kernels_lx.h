@@ -10,28 +10,23 @@
 // step is the one of kernels_cl.h with whole vectors in the lane: fields
 // pre-scaled by g = -gamma dt / (1 + alpha^2), the field's constant matrix A
 // (demagnetisation and anisotropy) applied as nine FMAs, the torque as
-// m x (h + alpha m x h), the binary32 stages as increments expanded about the
-// anchor, the length correction a polynomial that is tested once per block of
-// steps (RK4) or by one wave-uniform branch (Euler-Heun).  Against the general
-// form (kernels_ll.h), per wave step: RK4 372 -> 199 VALU instructions
-// (65,536-point PIMM sweep, 7.2e8 junction-steps, 20.9 -> 11.0 ms), Euler-Heun
-// 425 -> 254 (131,072 instances x 10,000 steps 24.9 -> 13.6 ms; a single wave
-// of instances 1.14 -> 0.5 us per step).
-// WPE: waves per SIMD the register allocation must leave room for.  The
-// ensembles run many waves per SIMD: 4 caps the kernel at 128 VGPRs (setup
-// spills to scratch there, the step loop does not).
+// m x (h + alpha m x h), the length correction a polynomial that is tested once
+// per block of steps (RK4) or by one wave-uniform branch (Euler-Heun).  RK4
+// steps are binary64 in either mode: a binary64 FMA issues as fast as a
+// binary32 one here, and stages in plain binary64 take 139 instructions a step
+// against 199 for binary32 increments about a binary64 anchor (33,000 points
+// 0.81 -> 0.62 ms, 196,608 points 2.10 -> 1.94 ms for 2,000 steps at most).
+// Against the general form (kernels_ll.h): RK4 372 -> 139 VALU instructions,
+// Euler-Heun 425 -> 254 (131,072 instances x 10,000 steps 24.9 -> 13.3 ms; a
+// single wave of instances 1.14 -> 0.5 us per step; in binary64 with the same
+// normals also 254, and more registers).
+// WPE: waves per SIMD the register allocation must leave room for.
 #pragma once
 
 #include "kernels_cl.h"
 
 namespace cmtj {
 
-template <class R>
-__device__ __forceinline__ V3<R> cross_add(V3<R> a, V3<R> b, V3<R> c, V3<R> d) {  // a x b + c x d
-  return mk<R>(fma(a.y, b.z, fma(-a.z, b.y, fma(c.y, d.z, -c.z * d.y))),
-               fma(a.z, b.x, fma(-a.x, b.z, fma(c.z, d.x, -c.x * d.z))),
-               fma(a.x, b.y, fma(-a.y, b.x, fma(c.x, d.y, -c.y * d.x))));
-}
 template <class R>
 __device__ __forceinline__ V3<R> cross_plus(V3<R> a, V3<R> b, V3<R> y) {  // a x b + y
   return mk<R>(fma(a.y, b.z, fma(-a.z, b.y, y.x)), fma(a.z, b.x, fma(-a.x, b.z, y.y)),
@@ -59,11 +54,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   static_assert(L == 2 || L == 4, "L lanes per instance must divide a 16-lane DPP row");
   static_assert(FM & F_EXACT, "exact feature sets");
   static_assert(!RK4 || !((FM & F_ALL) & ~(F_ANIS | F_IEC | F_DYNH)), "RK4: anisotropy, IEC, field drives");
-  static_assert(!RK4 || (FM & F_KSTEP), "RK4: step drives");
+  static_assert(!RK4 || ((FM & F_KSTEP) && sizeof(R) == 8), "RK4: step drives, binary64");
   static_assert(RK4 || (SOLVER == CMTJ_EULER_HEUN && !((FM & F_ALL) & ~(F_ANIS | F_DYN | F_SOT | F_THERMAL)) &&
                         (FM & F_KTRAP)),
                 "Euler-Heun: anisotropy, SOT, temperature, trapezoid drives of scalar slots");
-  constexpr bool F32 = sizeof(R) == 4;
   constexpr int NR = ND >= 0 ? ND : DREG;
   static_assert(NR <= DREG, "every record in registers");
   auto has_rec = [&](int r) { return ND >= 0 || r < g.ndyn; };
@@ -201,8 +195,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     }
   };
   const double jn = hasT ? jt : jb;  // L = 2: towards the other layer
-  const Mat3<float> Af{cvt<float>(A.r0), cvt<float>(A.r1), cvt<float>(A.r2)};
-  const float alphaf = (float)alpha;
   [[maybe_unused]] const Mat3<R> AR{cvt<R>(A.r0), cvt<R>(A.r1), cvt<R>(A.r2)};
   [[maybe_unused]] const V3<R> hbR = cvt<R>(hb);
   const R alphaR = (R)alpha;
@@ -256,28 +248,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         gg = axpy(alpha, cross(s, h), h);
         return cross(s, gg);
       };
-      if constexpr (F32) {
-        // rk4_step (core/junction.hpp:1017-1041): k1 in binary64, stages 2-4
-        // as binary32 increments about it
-        V3<double> h, gg;
-        const V3<double> k1 = torque(m, B, h, gg);
-        const V3<float> mf = cvt<float>(m), h0 = cvt<float>(h), g0 = cvt<float>(gg), k1f = cvt<float>(k1);
-        auto delta = [&](V3<float> d, V3<float> dd) __attribute__((always_inline)) -> V3<float> {
-          const V3<float> dh = Af.apply(d, dd), s = mf + d;
-          const V3<float> dg = axpy(alphaf, cross_add(s, dh, d, h0), dh);
-          return cross_add(s, dg, d, g0);
-        };
-        V3<float> dm = mk<float>(0, 0, 0), de = dm;
-        if constexpr (DRV != 0) {
-          dm = cvt<float>(drive(t + 0.5 * dt) - D0);
-          de = cvt<float>(drive(t + dt) - D0);
-        }
-        const V3<float> d2 = k1f * 0.5f;
-        const V3<float> k2 = delta(d2, dm);
-        const V3<float> k3 = delta(axpy(0.5f, k2, d2), dm);
-        const V3<float> k4 = delta(k1f + k3, de);
-        mn = m + axpy(1.0 / 6.0, cvt<double>(axpy(2.f, k2 + k3, k4)), k1);
-      } else {
+      // rk4_step (core/junction.hpp:1017-1041)
+      {
         V3<double> h, gg, Bm = B, Be = B;
         if constexpr (DRV != 0) {
           Bm = B + (drive(t + 0.5 * dt) - D0);
