@@ -344,6 +344,35 @@ static void signature(const cmtj_junction& j, const cmtj_layer* L, const std::ve
   for (const Rec& r : recs) sig.push_back(r.meta);
 }
 
+// Instance slot that holds no instance (pair_waves).
+constexpr uint32_t kNoInstance = 0xFFFFFFFFu;
+
+// Lays a group's waves (P instances each, longest first) out for workgroups
+// that hold a whole CU's share, where that gives every SIMD two or three: a
+// workgroup's waves go to the four SIMDs in turn, so waves w, w + 4, w + 8 of
+// one share a SIMD.  Rounds over the SIMDs alternate between ascending and
+// descending lengths, the last one descending, which levels the SIMDs' sums;
+// a short last round leaves slots without an instance.  As one-wave
+// workgroups, dealt longest first, the longest and the median wave share a
+// SIMD while others idle, and which waves share one depends on what the
+// dispatcher placed before (65,536-point PIMM sweep, 2,000 to 20,000 steps,
+// 2048 waves: 9.8 ms either way, paired within workgroups 7.4 ms).  Returns
+// the threads of a workgroup, 64 where the group is left as it is: one round
+// has nothing to pair, from four on waves start as others end and longest
+// first is the rule.
+static uint32_t pair_waves(std::vector<uint32_t>& ord, size_t P, int wg) {
+  const size_t waves = (ord.size() + P - 1) / P, rounds = (waves + kSimds - 1) / kSimds;
+  if (rounds < 2 || 4 * rounds > (size_t)wg) return 64;
+  std::vector<uint32_t> out(rounds * kSimds * P, kNoInstance);
+  for (size_t w = 0; w < waves; ++w) {
+    const size_t r = w / kSimds, q = w % kSimds, s = (rounds - 1 - r) % 2 == 0 ? q : kSimds - 1 - q;
+    const size_t at = (s / 4) * (4 * rounds) + r * 4 + s % 4;
+    std::copy(ord.begin() + w * P, ord.begin() + std::min(ord.size(), (w + 1) * P), out.begin() + at * P);
+  }
+  ord.swap(out);
+  return (uint32_t)(256 * rounds);
+}
+
 // Builds every group of a plan into one device arena obtained from `get`.
 // A group holds the junctions of one structure signature (layer count,
 // solver, log layout, per-layer modes, driver kinds and slots), so every
@@ -393,7 +422,8 @@ static int build_plan(cmtj_plan* P, const cmtj_junction* js, size_t n, const cmt
   const size_t G = sigs.size();
   std::vector<std::vector<uint32_t>> orders(G);
   std::vector<std::vector<DynRec>> nums(G);
-  std::vector<uint32_t> flags(G);
+  std::vector<uint32_t> flags(G), longest(G), threads(G, 64);
+  std::vector<const KEntry*> kernels(G);
   for (size_t g = 0; g < G; ++g) {
     std::vector<uint32_t>& ord = orders[g];
     ord = members[g];
@@ -401,15 +431,29 @@ static int build_plan(cmtj_plan* P, const cmtj_junction* js, size_t n, const cmt
     // dispatcher starts the long ones first
     std::stable_sort(ord.begin(), ord.end(),
                      [&](uint32_t a, uint32_t b) { return js[a].n_steps > js[b].n_steps; });
+    longest[g] = js[ord[0]].n_steps;
     uint32_t f = 0;
+    for (uint32_t i : ord) f |= junction_flags(js[i], layers + js[i].layer_offset);
+    flags[g] = f;
+    const cmtj_junction& j0 = js[ord[0]];
+    uint32_t kinds = 0;
+    for (const Rec& r : recs_of[ord[0]]) {
+      const int ty = r.meta & 0xff;
+      kinds |= (ty == CMTJ_STEP) ? KIND_STEP : (ty == CMTJ_SINE) ? KIND_SINE : (ty == CMTJ_TRAPEZOID) ? KIND_TRAP
+                                                                                               : KIND_OTHER;
+    }
+    kernels[g] = pick_kernel(prec, j0.n_layers, j0.solver, f, kinds, (int)recs_of[ord[0]].size(),
+                             (j0.log_mask & CMTJ_LOG_ENERGY) != 0,
+                             lanes == CMTJ_LANES_QUEUE ? (int)CMTJ_LANES_AUTO : lanes, ord.size(),
+                             (uint32_t)j0.log_mask | ((uint32_t)j0.mr_mode << 8) |
+                                 (log_dtype == CMTJ_LOG_F32 ? (1u << 16) : 0u));
+    if (!kernels[g]) return fail(CMTJ_ERR_INVALID, "no kernel for this junction configuration");
+    if (kernels[g]->wg && js[ord.back()].n_steps != longest[g])
+      threads[g] = pair_waves(ord, 64 / (size_t)kernels[g]->lpi, kernels[g]->wg);
     const size_t nd = recs_of[ord[0]].size();
     nums[g].resize(std::max<size_t>(nd, 1) * ord.size());
-    for (size_t p = 0; p < ord.size(); ++p) {
-      const cmtj_junction& j = js[ord[p]];
-      f |= junction_flags(j, layers + j.layer_offset);
-      for (size_t k = 0; k < nd; ++k) nums[g][k * ord.size() + p] = recs_of[ord[p]][k].num;
-    }
-    flags[g] = f;
+    for (size_t p = 0; p < ord.size(); ++p)
+      for (size_t k = 0; k < nd && ord[p] != kNoInstance; ++k) nums[g][k * ord.size() + p] = recs_of[ord[p]][k].num;
   }
   // arena layout
   size_t off = 0;
@@ -457,19 +501,7 @@ static int build_plan(cmtj_plan* P, const cmtj_junction* js, size_t n, const cmt
     if (upload(o_dyn[g], nums[g].data(), nums[g].size() * sizeof(DynRec))) return CMTJ_ERR_HIP;
     const cmtj_junction& j0 = js[orders[g][0]];
     const cmtj_layer* L0 = layers + j0.layer_offset;
-    const bool loge = (j0.log_mask & CMTJ_LOG_ENERGY) != 0;
-    uint32_t kinds = 0;
-    for (const Rec& r : recs_of[orders[g][0]]) {
-      const int ty = r.meta & 0xff;
-      kinds |= (ty == CMTJ_STEP) ? KIND_STEP : (ty == CMTJ_SINE) ? KIND_SINE : (ty == CMTJ_TRAPEZOID) ? KIND_TRAP
-                                                                                               : KIND_OTHER;
-    }
-    const KEntry* k = pick_kernel(prec, j0.n_layers, j0.solver, flags[g], kinds,
-                                  (int)recs_of[orders[g][0]].size(), loge,
-                                  lanes == CMTJ_LANES_QUEUE ? (int)CMTJ_LANES_AUTO : lanes, orders[g].size(),
-                                  (uint32_t)j0.log_mask | ((uint32_t)j0.mr_mode << 8) |
-                                      (log_dtype == CMTJ_LOG_F32 ? (1u << 16) : 0u));
-    if (!k) return fail(CMTJ_ERR_INVALID, "no kernel for this junction configuration");
+    const KEntry* k = kernels[g];
     Group Gr;
     Gr.k = k;
     std::memset(&Gr.a, 0, sizeof(Gr.a));
@@ -489,8 +521,9 @@ static int build_plan(cmtj_plan* P, const cmtj_junction* js, size_t n, const cmt
     for (int l = 0; l < j0.n_layers; ++l) Gr.a.lbits[l] = layer_bits(L0[l]);
     for (size_t q = 0; q < r0.size(); ++q) Gr.a.dmeta[q] = r0[q].meta;
     Gr.a.c = *c;
-    Gr.blocks = (uint32_t)(((uint64_t)Gr.a.n * (uint64_t)k->lpi + 63) / 64);
-    Gr.steps = j0.n_steps;  // longest first
+    Gr.threads = threads[g];
+    Gr.blocks = (uint32_t)(((uint64_t)Gr.a.n * (uint64_t)k->lpi + threads[g] - 1) / threads[g]);
+    Gr.steps = longest[g];
     if (lanes == CMTJ_LANES_QUEUE && j0.solver == CMTJ_DORMAND_PRINCE && j0.n_layers == 1) {
       Gr.queue = (uint32_t*)(arena + o_queue) + g;
       Gr.blocks = (std::min<uint32_t>(Gr.a.n, queue_lanes()) + 63) / 64;

@@ -4,10 +4,10 @@
 #include "registry.h"
 namespace cmtj {
 static const KEntry kE[] = {
-    CMTJ_KLX(double, CMTJ_FP32, 2, CMTJ_RK4, FM_PIMM, 1, -1),  // binary64 steps in either mode: see kernels_lx.h
-    CMTJ_KLX(double, CMTJ_FP64, 2, CMTJ_RK4, FM_PIMM, 1, -1),
-    CMTJ_KLX(double, CMTJ_FP32, 4, CMTJ_RK4, FM_PIMM, 1, -1),  // 3-4 layer IEC chains with a field step
-    CMTJ_KLX(double, CMTJ_FP64, 4, CMTJ_RK4, FM_PIMM, 1, -1),
+    CMTJ_KLX(double, CMTJ_FP32, 2, CMTJ_RK4, FM_PIMM, 3, -1),  // binary64 steps in either mode: see kernels_lx.h
+    CMTJ_KLX(double, CMTJ_FP64, 2, CMTJ_RK4, FM_PIMM, 3, -1),
+    CMTJ_KLX(double, CMTJ_FP32, 4, CMTJ_RK4, FM_PIMM, 3, -1),  // 3-4 layer IEC chains with a field step
+    CMTJ_KLX(double, CMTJ_FP64, 4, CMTJ_RK4, FM_PIMM, 3, -1),
     CMTJ_KE(float, CMTJ_FP32, 2, CMTJ_RK4, FM_PIMM, false),
     CMTJ_KE(double, CMTJ_FP64, 2, CMTJ_RK4, FM_PIMM, false),
     CMTJ_KE(float, CMTJ_FP32, 1, CMTJ_RK4, FM_RH, false),

@@ -47,9 +47,11 @@ struct Mat3 {
 };
 
 // ND: number of time-dependent records when fixed at compile time, -1 to read
-// it from the group.
+// it from the group.  RK4: workgroups of up to 4 WPE waves (see pair_waves in
+// engine.hip).
 template <class R, int L, int SOLVER, uint32_t FM, int WPE = 1, int ND = -1>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void k_junction_lx(GroupArgs g) {
+__global__ __launch_bounds__(SOLVER == CMTJ_RK4 ? 256 * WPE : 64) __attribute__((amdgpu_waves_per_eu(WPE))) void
+k_junction_lx(GroupArgs g) {
   constexpr bool RK4 = SOLVER == CMTJ_RK4;
   static_assert(L == 2 || L == 4, "L lanes per instance must divide a 16-lane DPP row");
   static_assert(FM & F_EXACT, "exact feature sets");
@@ -69,6 +71,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   const bool act = ly < nl;
   const int lyr = act ? ly : 0;  // idle lanes shadow layer 0 and write nothing
   const uint32_t jid = g.order[inst];
+  if (jid == 0xFFFFFFFFu) return;  // a slot without an instance (pair_waves)
   const cmtj_junction* J = g.js + jid;
   const uint32_t nsteps = J->n_steps;
   const uint32_t W = J->write_every;

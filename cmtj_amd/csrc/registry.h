@@ -16,6 +16,7 @@ struct KEntry {
   const char* name;
   int nd1;  // 1 + the number of time-dependent records the kernel is compiled for; 0: any
   int logf;  // 0: any log layout; 1: m_x of every layer + classic R, binary32 entries
+  int wg;    // waves a workgroup may hold, instance slots without an instance allowed; 0: one, none
 };
 
 struct KTable {
@@ -77,7 +78,8 @@ KTable kernels_group_cl();  // Kanao / Nomura groups on one lane per component
 // the large batches' exact sets (kernels_lx.h), the register allocation capped for WPE waves per SIMD
 #define CMTJ_KLX(R, PREC, L, S, FM, WPE, ND)                                                \
   {PREC, L, L, S, FM, false, (const void*)&cmtj::k_junction_lx<R, L, S, FM, WPE, ND>,       \
-   "k_junction_ll<" #R "," #L "," #S "," #FM "," #ND ",waves " #WPE ">", (ND) + 1}
+   "k_junction_ll<" #R "," #L "," #S "," #FM "," #ND ",waves " #WPE ">", (ND) + 1, 0,       \
+   (S) == CMTJ_RK4 ? 4 * (WPE) : 0}
 
 #define CMTJ_KC(L, FM, ND)                                                                     \
   {CMTJ_FP32, L, 4 * (L), CMTJ_RK4, FM, false, (const void*)&cmtj::k_junction_cl<L, FM, ND>,  \
