@@ -160,68 +160,73 @@ __device__ __forceinline__ T cross_a(const Rot<T>& x, T yb, T yc) {
 // the step's layout).
 #define CL_ROT1 "quad_perm:[1,2,0,3] row_mask:0xf bank_mask:0xf\n\t"
 #define CL_ROT2 "quad_perm:[2,0,1,3] row_mask:0xf bank_mask:0xf\n\t"
+#define CL_STAGES(OFF) \
+  "v_mul_f32 %[d], 0.5, %[k1]\n\t" \
+  "v_cvt_f32_f64 %[g1], %[gb]\n\t" \
+  "v_fma_f32 %[h], %[a0], %[d], %[dm]\n\t" \
+  OFF \
+  "v_add_f32_dpp %[s1], %[d], %[m1] " CL_ROT1 \
+  "v_add_f32_dpp %[s2], %[d], %[m2] " CL_ROT2 \
+  "v_mul_f32_dpp %[p], %[d], %[h2] " CL_ROT1 \
+  "v_fmac_f32_dpp %[p], %[d], -%[h1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[p], %[h], %[s1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[p], %[h], -%[s2] " CL_ROT1 \
+  "v_fmac_f32 %[h], %[al], %[p]\n\t" \
+  "v_cvt_f32_f64 %[g2], %[gc]\n\t" \
+  "v_mul_f32_dpp %[r], %[d], %[g2] " CL_ROT1 \
+  "v_fmac_f32_dpp %[r], %[d], -%[g1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[r], %[h], %[s1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[r], %[h], -%[s2] " CL_ROT1 \
+  "v_fmac_f32 %[d], 0.5, %[r]\n\t" \
+  "v_add_f32 %[acc], %[r], %[r]\n\t" \
+  "v_fma_f32 %[h], %[a0], %[d], %[dm]\n\t" \
+  OFF \
+  "v_add_f32_dpp %[s1], %[d], %[m1] " CL_ROT1 \
+  "v_add_f32_dpp %[s2], %[d], %[m2] " CL_ROT2 \
+  "v_mul_f32_dpp %[p], %[d], %[h2] " CL_ROT1 \
+  "v_fmac_f32_dpp %[p], %[d], -%[h1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[p], %[h], %[s1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[p], %[h], -%[s2] " CL_ROT1 \
+  "v_fmac_f32 %[h], %[al], %[p]\n\t" \
+  "v_mul_f32_dpp %[r], %[d], %[g2] " CL_ROT1 \
+  "v_fmac_f32_dpp %[r], %[d], -%[g1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[r], %[h], %[s1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[r], %[h], -%[s2] " CL_ROT1 \
+  "v_add_f32 %[d], %[k1], %[r]\n\t" \
+  "v_fmac_f32 %[acc], 2.0, %[r]\n\t" \
+  "v_fma_f32 %[h], %[a0], %[d], %[de]\n\t" \
+  OFF \
+  "v_add_f32_dpp %[s1], %[d], %[m1] " CL_ROT1 \
+  "v_add_f32_dpp %[s2], %[d], %[m2] " CL_ROT2 \
+  "v_mul_f32_dpp %[p], %[d], %[h2] " CL_ROT1 \
+  "v_fmac_f32_dpp %[p], %[d], -%[h1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[p], %[h], %[s1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[p], %[h], -%[s2] " CL_ROT1 \
+  "v_fmac_f32 %[h], %[al], %[p]\n\t" \
+  "v_mul_f32_dpp %[r], %[d], %[g2] " CL_ROT1 \
+  "v_fmac_f32_dpp %[r], %[d], -%[g1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[r], %[h], %[s1] " CL_ROT2 \
+  "v_fmac_f32_dpp %[r], %[h], -%[s2] " CL_ROT1 \
+  "v_add_f32 %[acc], %[acc], %[r]"
+#define CL_STAGE_OPERANDS \
+  : [d] "=&v"(d), [g1] "=&v"(g1), [g2] "=&v"(g2), [h] "=&v"(h), [s1] "=&v"(s1), [s2] "=&v"(s2), [p] "=&v"(p), \
+  [r] "=&v"(r), [acc] "=&v"(acc) \
+  : [k1] "v"(k1), [a0] "v"(K.a0), [a1] "v"(K.a1), [a2] "v"(K.a2), [al] "v"(K.al), [m1] "v"(m1), [m2] "v"(m2), \
+  [h1] "v"(h1), [h2] "v"(h2), [gb] "v"(gb), [gc] "v"(gc), [dm] "v"(dmid), [de] "v"(dend)
 struct StageConst {
   float a0, a1, a2, al;  // the field matrix's row against components c, c + 1, c + 2; alpha
 };
+template <bool DG>
 __device__ __forceinline__ float stage_increments(const StageConst& K, float k1, const Rot<double>& m,
                                                   const Rot<double>& h0, double gb, double gc, float dmid,
                                                   float dend) {
   const float m1 = (float)m.b, m2 = (float)m.c, h1 = (float)h0.b, h2 = (float)h0.c;
   float d, g1, g2, h, s1, s2, p, r, acc;
-  asm("v_mul_f32 %[d], 0.5, %[k1]\n\t"
-      "v_cvt_f32_f64 %[g1], %[gb]\n\t"
-      "v_fma_f32 %[h], %[a0], %[d], %[dm]\n\t"
-      "v_fmac_f32_dpp %[h], %[d], %[a1] " CL_ROT1
-      "v_fmac_f32_dpp %[h], %[d], %[a2] " CL_ROT2
-      "v_add_f32_dpp %[s1], %[d], %[m1] " CL_ROT1
-      "v_add_f32_dpp %[s2], %[d], %[m2] " CL_ROT2
-      "v_mul_f32_dpp %[p], %[d], %[h2] " CL_ROT1
-      "v_fmac_f32_dpp %[p], %[d], -%[h1] " CL_ROT2
-      "v_fmac_f32_dpp %[p], %[h], %[s1] " CL_ROT2
-      "v_fmac_f32_dpp %[p], %[h], -%[s2] " CL_ROT1
-      "v_fmac_f32 %[h], %[al], %[p]\n\t"
-      "v_cvt_f32_f64 %[g2], %[gc]\n\t"
-      "v_mul_f32_dpp %[r], %[d], %[g2] " CL_ROT1
-      "v_fmac_f32_dpp %[r], %[d], -%[g1] " CL_ROT2
-      "v_fmac_f32_dpp %[r], %[h], %[s1] " CL_ROT2
-      "v_fmac_f32_dpp %[r], %[h], -%[s2] " CL_ROT1
-      "v_fmac_f32 %[d], 0.5, %[r]\n\t"
-      "v_add_f32 %[acc], %[r], %[r]\n\t"
-      "v_fma_f32 %[h], %[a0], %[d], %[dm]\n\t"
-      "v_fmac_f32_dpp %[h], %[d], %[a1] " CL_ROT1
-      "v_fmac_f32_dpp %[h], %[d], %[a2] " CL_ROT2
-      "v_add_f32_dpp %[s1], %[d], %[m1] " CL_ROT1
-      "v_add_f32_dpp %[s2], %[d], %[m2] " CL_ROT2
-      "v_mul_f32_dpp %[p], %[d], %[h2] " CL_ROT1
-      "v_fmac_f32_dpp %[p], %[d], -%[h1] " CL_ROT2
-      "v_fmac_f32_dpp %[p], %[h], %[s1] " CL_ROT2
-      "v_fmac_f32_dpp %[p], %[h], -%[s2] " CL_ROT1
-      "v_fmac_f32 %[h], %[al], %[p]\n\t"
-      "v_mul_f32_dpp %[r], %[d], %[g2] " CL_ROT1
-      "v_fmac_f32_dpp %[r], %[d], -%[g1] " CL_ROT2
-      "v_fmac_f32_dpp %[r], %[h], %[s1] " CL_ROT2
-      "v_fmac_f32_dpp %[r], %[h], -%[s2] " CL_ROT1
-      "v_add_f32 %[d], %[k1], %[r]\n\t"
-      "v_fmac_f32 %[acc], 2.0, %[r]\n\t"
-      "v_fma_f32 %[h], %[a0], %[d], %[de]\n\t"
-      "v_fmac_f32_dpp %[h], %[d], %[a1] " CL_ROT1
-      "v_fmac_f32_dpp %[h], %[d], %[a2] " CL_ROT2
-      "v_add_f32_dpp %[s1], %[d], %[m1] " CL_ROT1
-      "v_add_f32_dpp %[s2], %[d], %[m2] " CL_ROT2
-      "v_mul_f32_dpp %[p], %[d], %[h2] " CL_ROT1
-      "v_fmac_f32_dpp %[p], %[d], -%[h1] " CL_ROT2
-      "v_fmac_f32_dpp %[p], %[h], %[s1] " CL_ROT2
-      "v_fmac_f32_dpp %[p], %[h], -%[s2] " CL_ROT1
-      "v_fmac_f32 %[h], %[al], %[p]\n\t"
-      "v_mul_f32_dpp %[r], %[d], %[g2] " CL_ROT1
-      "v_fmac_f32_dpp %[r], %[d], -%[g1] " CL_ROT2
-      "v_fmac_f32_dpp %[r], %[h], %[s1] " CL_ROT2
-      "v_fmac_f32_dpp %[r], %[h], -%[s2] " CL_ROT1
-      "v_add_f32 %[acc], %[acc], %[r]"
-      : [d] "=&v"(d), [g1] "=&v"(g1), [g2] "=&v"(g2), [h] "=&v"(h), [s1] "=&v"(s1), [s2] "=&v"(s2), [p] "=&v"(p),
-        [r] "=&v"(r), [acc] "=&v"(acc)
-      : [k1] "v"(k1), [a0] "v"(K.a0), [a1] "v"(K.a1), [a2] "v"(K.a2), [al] "v"(K.al), [m1] "v"(m1), [m2] "v"(m2),
-        [h1] "v"(h1), [h2] "v"(h2), [gb] "v"(gb), [gc] "v"(gc), [dm] "v"(dmid), [de] "v"(dend));
+  if constexpr (DG)
+    asm(CL_STAGES("") CL_STAGE_OPERANDS);
+  else
+    asm(CL_STAGES("v_fmac_f32_dpp %[h], %[d], %[a1] " CL_ROT1 "v_fmac_f32_dpp %[h], %[d], %[a2] " CL_ROT2)
+            CL_STAGE_OPERANDS);
   return acc;
 }
 
@@ -361,10 +366,10 @@ __device__ __forceinline__ void lds_barrier() {
 // stage's m) is all that crosses lanes; the LLG torque is m x (h + alpha m x h)
 // with the field pre-scaled; the length correction is a polynomial (a
 // binary64 square root and division took a quarter of a binary64 step).
-// Measured before and after: R(H) loop, 101 one-layer instances x 50,000
-// binary64 steps 21.5 -> 12.5 ms; 512 oscillators x 50,000 steps 44.2 -> 15.4
-// ms; 1023 one-layer instances under a sine field x 10,000 steps 14.9 -> 3.1
-// ms (three binary64 sines a step before, see Osc).
+// Measured before and after all of it: R(H) loop, 101 one-layer instances x
+// 50,000 binary64 steps 21.4 -> 10.0 ms; 512 oscillators x 50,000 steps 44.1 ->
+// 10.7 ms; 1023 one-layer instances under a sine field x 10,000 steps 14.9 ->
+// 2.6 ms (three binary64 sines a step before, see Osc).
 template <int L, uint32_t FM, int ND, bool F64 = false, int SOLVER = CMTJ_RK4, int LOGF = 0, bool STK = false,
           int GW = 0, bool NF = false>
 __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArgs g) {
@@ -549,6 +554,27 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
     K.kick = P.gconv * sqrt(dt);
     K.sg0 = K.therm ? sqrt(K.sig2 * K.bT) * K.kick : z;
   }
+  // A multiple of m added to the field changes no torque, so a lane takes the
+  // matrix less the identity times its row c + 1's diagonal entry, which that
+  // row then has no more (binary32 increments share their field between lanes
+  // and stay as they are, and so do the stochastic solvers, whose one field a
+  // step gains nothing).
+  constexpr bool GAUGE = F64 && SOLVER == CMTJ_RK4;
+  if constexpr (GAUGE) {
+    const double lam = K.A1.b;
+    K.A0.a -= lam;
+    K.A1.b = 0.0;
+    K.A2.c -= lam;
+  }
+  // Anisotropy along an axis and a diagonal demagnetising tensor, in every lane
+  // of the wave: the matrix is diagonal, and a field evaluation takes two FMAs
+  // instead of eight (binary32 increments: one instead of three).  Decided per
+  // wave, with the same bits either way (a zero entry adds a zero).  Before and
+  // after: R(H) loop 12.6 -> 10.0 ms, PIMM sweep 44.6 -> 40.4 ms, oscillators
+  // 13.2 -> 10.7 ms, sine field 3.0 -> 2.6 ms.
+  constexpr bool DGSET = SOLVER == CMTJ_RK4 && !(FM & (F_DEMAG_OFF | F_IEC2));
+  const bool diag = DGSET && __ballot(K.A0.b != 0.0 || K.A0.c != 0.0 || K.A1.a != 0.0 || K.A1.c != 0.0 ||
+                                      K.A2.a != 0.0 || K.A2.b != 0.0) == 0ull;
   // eta's denominator is lam2 + 1 on every STT lane of the wave (lambda = 1,
   // the usual spacer): the torque then needs no division
   const bool den_const = (FM & F_STT) != 0 && __ballot(K.stt && (K.alt || K.lam2 != 1.0)) == 0ull;
@@ -1005,7 +1031,8 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   char* pk = lpl;          // the lane's next entry
   double lv = 0.0;
   auto step = [&](auto drv_tag, auto log_tag, auto chk_tag) __attribute__((always_inline)) {
-    constexpr bool DRV = decltype(drv_tag)::value;
+    constexpr bool DRV = (decltype(drv_tag)::value & 1) != 0;
+    constexpr bool DG = (decltype(drv_tag)::value & 2) != 0;
     constexpr int LOGM = decltype(log_tag)::value;
     constexpr bool CHK = decltype(chk_tag)::value;
     constexpr bool DRIVEN = DRV && (FM & (F_DYN | F_DYNH)) != 0;
@@ -1192,7 +1219,13 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       auto along = [&](const Rot<double>& r, double x) {
         return fma(r.c, s.c, fma(r.b, s.b, fma(r.a, s.a, x)));
       };
-      Rot<double> h{along(A.a, B.a), along(A.b, B.b), along(A.c, B.c)};
+      Rot<double> h;
+      if constexpr (DG)
+        h = {fma(A.a.a, s.a, B.a), GAUGE ? B.b : fma(A.b.b, s.b, B.b), fma(A.c.c, s.c, B.c)};
+      else if constexpr (GAUGE && !(FM & F_IEC2))
+        h = {along(A.a, B.a), fma(A.b.c, s.c, fma(A.b.a, s.a, B.b)), along(A.c, B.c)};
+      else
+        h = {along(A.a, B.a), along(A.b, B.b), along(A.c, B.c)};
       if constexpr ((FM & (F_DYN | F_ANIS2)) != 0) {
         if (CMTJ_HAS(F_ANIS2) || k_driven) {
           // calculateSecondOrderAnisotropy (:645-652): 4 K2 (anis . m)^3 / Ms,
@@ -1373,7 +1406,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         turn();
         dend = (float)(drive(FTT, t + dt, 2, b0, nb).H - d0.H);
       }
-      mn = m.a + fma((double)stage_increments(KF, (float)k1, m, h, gb, gc, dmid, dend), 1.0 / 6.0, k1);
+      mn = m.a + fma((double)stage_increments<DG>(KF, (float)k1, m, h, gb, gc, dmid, dend), 1.0 / 6.0, k1);
     }
     // ---- CVector::normalize (core/cvector.hpp:185-192).  Binary64: |m|^2 - 1
     // as a butterfly over the quad, (x^2 + y^2) + (z^2 - 1) in all its lanes,
@@ -1670,6 +1703,10 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       }
     }
   };
+  auto run = [&](auto dg_tag) __attribute__((always_inline)) {
+  constexpr int DG2 = decltype(dg_tag)::value ? 2 : 0;
+  constexpr std::integral_constant<int, DG2> OFF{};
+  constexpr std::integral_constant<int, DG2 + 1> ON{};
   if constexpr ((FM & F_KSTEP) != 0 && !(FM & F_TABLE)) {
     // steps [ia, ib) may meet a record's window [win_lo, win_hi]; every
     // stage time of a step before ia is below win_lo, of a step from ib on
@@ -1680,11 +1717,20 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       ia = a <= (double)i ? i : (a >= (double)iend ? iend : (uint32_t)a);
       ib = b <= (double)ia ? ia : (b >= (double)iend ? iend : (uint32_t)b);
     }
-    phase(ia, std::false_type{});
-    phase(ib, std::true_type{});
-    phase(iend, std::false_type{});
+    phase(ia, OFF);
+    phase(ib, ON);
+    phase(iend, OFF);
   } else {
-    phase(iend, std::true_type{});
+    phase(iend, ON);
+  }
+  };
+  if constexpr (DGSET) {
+    if (diag)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
+  } else {
+    run(std::false_type{});
   }
   if (g.mag_out && live) g.mag_out[((size_t)jid * CMTJ_MAX_LAYERS + ly) * 3 + c] = m.a;
   if (g.status && own && q == 0) {
