@@ -125,9 +125,9 @@ static const KEntry* pick_kernel(int prec, int nl, int solver, uint32_t flags, u
   // automatic choice: on a batch too small to fill the chip, the time of a
   // sweep is its longest instance's step count times the latency of one
   // wave step.  One lane per component issues about half the instructions
-  // per wave step of one lane per layer (111 against 199 VALU on the PIMM
-  // set), at four times the lanes: it wins while its waves still fit one per
-  // SIMD, and costs about twice the instructions per junction-step beyond that
+  // per wave step of one lane per layer, and at four times the lanes spreads
+  // over more SIMDs (PIMM set: 94 against 111 VALU a step): it wins while its waves still fit one per
+  // SIMD, and costs several times the instructions per junction-step beyond that
   // (FP32 Euler-Heun, us per step: 8,192 two-layer switching devices 0.41
   // against 0.53, 16,384 0.65 against 0.55; 4,096 four-layer chains 0.90
   // against 1.09, 8,192 1.74 against 1.18).
@@ -135,8 +135,8 @@ static const KEntry* pick_kernel(int prec, int nl, int solver, uint32_t flags, u
   // one lane per layer for multilayer instances: its register footprint is
   // smaller than one lane per instance's, so more waves fit per SIMD, and the
   // exact sets of large batches have their leanest kernels there (65,536-point
-  // PIMM sweep 6.5e10 junction-steps/s against 2.4e10 with one lane per
-  // instance, 131,072-instance CIMS ensemble 9.6e10 against 6.3e10).
+  // PIMM sweep 1.1e11 junction-steps/s against 2.4e10 with one lane per
+  // instance, 131,072-instance CIMS ensemble 9.8e10 against 6.3e10).
   if (best[1] && (nl >= 2 || !best[0])) return best[1];
   if (best[0]) return best[0];
   return best[1] ? best[1] : best[2];

@@ -15,9 +15,10 @@
 // steps are binary64 in either mode: a binary64 FMA issues as fast as a
 // binary32 one here, and stages in plain binary64 take 139 instructions a step
 // against 199 for binary32 increments about a binary64 anchor (33,000 points
-// 0.81 -> 0.62 ms, 196,608 points 2.10 -> 1.94 ms for 2,000 steps at most).
-// Against the general form (kernels_ll.h): RK4 372 -> 139 VALU instructions,
-// Euler-Heun 425 -> 254 (131,072 instances x 10,000 steps 24.9 -> 13.3 ms; a
+// 0.81 -> 0.62 ms, 196,608 points 2.10 -> 1.94 ms for 2,000 steps at most),
+// and with a diagonal field matrix 111 (65,536 points, 2,000 to 20,000 steps,
+// 7.4 -> 6.7 ms).  Against the general form (kernels_ll.h): RK4 372 -> 111 VALU
+// instructions (20.7 -> 6.7 ms with the waves paired), Euler-Heun 425 -> 254 (131,072 instances x 10,000 steps 24.9 -> 13.3 ms; a
 // single wave of instances 1.14 -> 0.5 us per step; in binary64 with the same
 // normals also 254, and more registers).
 // WPE: waves per SIMD the register allocation must leave room for.
@@ -142,6 +143,19 @@ k_junction_lx(GroupArgs g) {
       nu = nsd * (R)sqrt(sig2 * bT);
     }
   }
+  // RK4: the matrix less the identity times its last diagonal entry (a multiple
+  // of m in the field moves nothing), and whether it is diagonal in every lane
+  // of the wave: two FMAs a field evaluation instead of eight, the same bits
+  // either way (as in kernels_cl.h)
+  bool diag = false;
+  if constexpr (RK4) {
+    const double lam = A.r2.z;
+    A.r0.x -= lam;
+    A.r1.y -= lam;
+    A.r2.z = 0.0;
+    diag = __ballot(A.r0.y != 0.0 || A.r0.z != 0.0 || A.r1.x != 0.0 || A.r1.z != 0.0 || A.r2.x != 0.0 ||
+                    A.r2.y != 0.0) == 0ull;
+  }
   // ---- drive records
   DynRec dr[DREG];
   bool on[DREG];
@@ -213,7 +227,8 @@ k_junction_lx(GroupArgs g) {
   // window, 1 inside, 2 every trapezoid on one line through the block.
   double lc[DREG] = {0.0, 0.0}, lt[DREG] = {0.0, 0.0}, la[DREG] = {0.0, 0.0};  // la + lc (t - lt)
   auto step = [&](auto drv_tag, auto log_tag, auto chk_tag) __attribute__((always_inline)) {
-    constexpr int DRV = decltype(drv_tag)::value;
+    constexpr int DRV = decltype(drv_tag)::value & 3;
+    constexpr bool DG = (decltype(drv_tag)::value & 4) != 0;
     constexpr int LOGM = decltype(log_tag)::value;
     constexpr bool CHK = decltype(chk_tag)::value;
     const double t = (double)i * dt;
@@ -247,7 +262,12 @@ k_junction_lx(GroupArgs g) {
         }
       }
       auto torque = [&](V3<double> s, V3<double> Bs, V3<double>& h, V3<double>& gg) __attribute__((always_inline)) {
-        h = A.apply(s, Bs);
+        if constexpr (DG)
+          h = mk<double>(fma(A.r0.x, s.x, Bs.x), fma(A.r1.y, s.y, Bs.y), Bs.z);
+        else
+          h = mk<double>(fma(A.r0.z, s.z, fma(A.r0.y, s.y, fma(A.r0.x, s.x, Bs.x))),
+                         fma(A.r1.z, s.z, fma(A.r1.y, s.y, fma(A.r1.x, s.x, Bs.y))),
+                         fma(A.r2.y, s.y, fma(A.r2.x, s.x, Bs.z)));
         gg = axpy(alpha, cross(s, h), h);
         return cross(s, gg);
       };
@@ -485,9 +505,15 @@ k_junction_lx(GroupArgs g) {
       ia = a <= (double)i ? i : (a >= (double)iend ? iend : (uint32_t)a);
       ib = b <= (double)ia ? ia : (b >= (double)iend ? iend : (uint32_t)b);
     }
-    phase(ia, C0{});
-    phase(ib, C1{});
-    phase(iend, C0{});
+    auto run = [&](auto off, auto on) __attribute__((always_inline)) {
+      phase(ia, off);
+      phase(ib, on);
+      phase(iend, off);
+    };
+    if (diag)
+      run(std::integral_constant<int, 4>{}, std::integral_constant<int, 5>{});
+    else
+      run(C0{}, C1{});
   } else {
     phase(iend, C1{});
   }

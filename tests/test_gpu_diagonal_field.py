@@ -1,4 +1,4 @@
-"""Component lanes with a diagonal field matrix (anisotropy along an axis) and
+"""Component and layer lanes with a diagonal field matrix (anisotropy along an axis) and
 with a full one: each against the oracle, and an instance's bits the same
 whether its wave holds tilted axes beside it or not.  Tolerances: the
 drop-in's bar in FP64, the bulk mode's in FP32."""
@@ -42,14 +42,16 @@ def _junction(nl, q, tilted, stt):
 
 
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
-@pytest.mark.parametrize("nl,stt", [(1, False), (2, False), (4, False), (2, True)])
-def test_axes(nl, stt, precision):
+@pytest.mark.parametrize("nl,stt,lanes", [(1, False, "per_component"), (2, False, "per_component"),
+                                          (4, False, "per_component"), (2, True, "per_component"),
+                                          (2, False, "per_layer"), (4, False, "per_layer")])
+def test_axes(nl, stt, lanes, precision):
     out = {}
     for tilted in (False, True):
         js = [_junction(nl, q, tilted, stt) for q in range(16)]
         b = JunctionBatch.from_junctions(js, 2.005e-11, 1e-13, 1e-13, SolverMode.RK4, precision=precision, log="m",
-                                         log_dtype="f64").set_lanes("per_component")
-        assert "k_junction_cl" in b.plan().info.kernel_name.decode() and b.plan().info.n_kernels == 1
+                                         log_dtype="f64").set_lanes(lanes)
+        assert ("k_junction_cl" if lanes == "per_component" else "waves 3") in b.plan().info.kernel_name.decode() and b.plan().info.n_kernels == 1
         r = b.run()
         olog, omag, _ = oracle.run_batch(b.js, b.layers, _lib.constants_get(), b.tables, b.log_elements)
         worst = float(np.max(np.abs(r.log.cpu().numpy() - olog)))
@@ -59,5 +61,5 @@ def test_axes(nl, stt, precision):
     # alone (or among axis-aligned ones) and beside tilted axes
     b, m = out[True]
     for q in (0, 1, 2, 5):
-        a = b.subset(np.array([q])).set_lanes("per_component")
+        a = b.subset(np.array([q])).set_lanes(lanes)
         np.testing.assert_array_equal(a.run().final_m.cpu().numpy()[0, :nl], m[q, :nl])
