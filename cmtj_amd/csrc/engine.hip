@@ -60,6 +60,7 @@ constexpr uint32_t kLogPimm = (CMTJ_LOG_MX | CMTJ_LOG_MR) | (CMTJ_MR_CLASSIC << 
 
 static bool covers(const KEntry& k, uint32_t flags, uint32_t kinds, int ndyn, uint32_t logcfg = 0xffffffffu) {
   if (k.logf == 1 && logcfg != kLogPimm) return false;
+  if (k.logf == 2 && !(logcfg & (1u << 16))) return false;
   const uint32_t feat = k.fm & F_ALL;
   if ((feat & flags) != flags) return false;
   if ((k.fm & F_EXACT) && (feat != flags || ndyn > DREG)) return false;  // exact kernels keep every record in registers

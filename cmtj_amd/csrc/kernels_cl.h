@@ -343,7 +343,8 @@ __device__ __forceinline__ void lds_barrier() {
 // ND: number of time-dependent records when fixed at compile time (exact
 // kernels), -1 to read it from the group.  F64: every stage in binary64
 // (the drop-in's arithmetic) instead of the anchored binary32 increments.
-// LOGF: 0 reads the log layout from the group; 1 compiles in m_x of every
+// LOGF: 0 reads the log layout from the group, 2 too but of binary32 entries;
+// 1 compiles in m_x of every
 // layer, the classic resistance and binary32 entries (the PIMM sweep's log).
 // STK: the instances are members of electrically coupled stacks
 // (Stack<T>::runSimulationKCL / runSimulationNonKCL with delayed coupling,
@@ -374,7 +375,7 @@ template <int L, uint32_t FM, int ND, bool F64 = false, int SOLVER = CMTJ_RK4, i
           int GW = 0, bool NF = false>
 __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArgs g) {
   // the compiled-in layout's R is layer 0 against layer 1
-  static_assert(LOGF == 0 || (L == 2 && (FM & F_EXACT) && (FM & F_IEC)), "two coupled layers");
+  static_assert(LOGF != 1 || (L == 2 && (FM & F_EXACT) && (FM & F_IEC)), "two coupled layers");
   static_assert(!STK || (F64 && LOGF == 0 && !(FM & F_KSTEP)),
                 "stacks: binary64, the group's log layout, every step through the same code");
   static_assert(!NF || (F64 && SOLVER != CMTJ_RK4 && (FM & F_THERMAL)), "binary32 normals: stochastic solvers");
@@ -391,7 +392,9 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   constexpr int LPI = 4 * L;
   constexpr int NN = (L == 1) ? 0 : (L == 2) ? 1 : 2;  // neighbours of a layer: none, the other one, top and bottom
   constexpr bool DYNS = (FM & F_DYN) != 0;              // time-dependent scalar slots
-  constexpr bool OSC = (FM & (F_DYN | F_DYNH)) != 0 && !(FM & (F_KSTEP | F_KTRAP));
+  // sine phases carried from stage to stage (binary32 increments logged in
+  // binary64 keep their single-precision waveforms, see PLAIN32)
+  constexpr bool OSC = (F64 || LOGF == 2) && (FM & (F_DYN | F_DYNH)) != 0 && !(FM & (F_KSTEP | F_KTRAP));
   const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t inst;
   int q;
@@ -575,6 +578,29 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   constexpr bool DGSET = SOLVER == CMTJ_RK4 && !(FM & (F_DEMAG_OFF | F_IEC2));
   const bool diag = DGSET && __ballot(K.A0.b != 0.0 || K.A0.c != 0.0 || K.A1.a != 0.0 || K.A1.c != 0.0 ||
                                       K.A2.a != 0.0 || K.A2.b != 0.0) == 0ull;
+  // Binary32 sets that take waveforms keep the form of their increments and
+  // their single-precision waveforms where entries are binary64, in which
+  // another order of the binary32 operations shows (3e-9 of m after 5,000
+  // steps); with binary32 entries they take the shorter ones (LOGF 2; a sine
+  // field's step 1.3 -> 0.3 us).
+  constexpr bool PLAIN32 = !F64 && LOGF != 2 && !(FM & F_KSTEP);
+  [[maybe_unused]] float p_an = 0, p_an1 = 0, p_an2 = 0, p_nms = 0, p_ak = 0, p_al = 0, p_g = 0;
+  [[maybe_unused]] double ig = 0.0;
+  if constexpr (PLAIN32) {
+    LP<double> P;
+    DV<double> base;
+    V3<double> m3;
+    load_layer<double>(g.layers[J->layer_offset + lyr], g.c, P, base, m3);
+    p_an = (float)K.an0;
+    p_an1 = (float)K.an1;
+    p_an2 = (float)K.an2;
+    const V3<double> nd = mk<double>(P.N[0], P.N[4], P.N[8]);
+    p_nms = live ? (float)(comp(nd, c) * P.ms_mu0) : 0.f;
+    p_ak = (float)(K.an0 * ((2.0 * base.K) * P.inv_ms));
+    p_al = (float)P.alpha;
+    p_g = (float)P.gconv * (float)dt;
+    ig = 1.0 / K.g;
+  }
   // eta's denominator is lam2 + 1 on every STT lane of the wave (lambda = 1,
   // the usual spacer): the torque then needs no division
   const bool den_const = (FM & F_STT) != 0 && __ballot(K.stt && (K.alt || K.lam2 != 1.0)) == 0ull;
@@ -1397,16 +1423,41 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       const double gb = fma(K.alpha, cross_b(m, h), h.b), gc = fma(K.alpha, cross_c2(m, h), h.c);
       const double k1 = cross_a(m, gb, gc);
       // ---- stages 2-4: binary32 increments about the anchor
-      const StageConst KF{(float)K.A0.a, (float)K.A0.b, (float)K.A0.c, (float)K.alpha};
       float dmid = 0.f, dend = 0.f;
       if constexpr (DRIVEN) {
-        // scaled drive increments against the start of the step
+        // drive increments against the start of the step
+        const double u = PLAIN32 ? ig : 1.0;
         turn();
-        dmid = (float)(drive(FTT, t + 0.5 * dt, 1, b0, nb).H - d0.H);
+        dmid = (float)((drive(FTT, t + 0.5 * dt, 1, b0, nb).H - d0.H) * u);
         turn();
-        dend = (float)(drive(FTT, t + dt, 2, b0, nb).H - d0.H);
+        dend = (float)((drive(FTT, t + dt, 2, b0, nb).H - d0.H) * u);
       }
-      mn = m.a + fma((double)stage_increments<DG>(KF, (float)k1, m, h, gb, gc, dmid, dend), 1.0 / 6.0, k1);
+      if constexpr (PLAIN32) {
+        // unscaled, cross products expanded about the anchor: (m0 + d) x (H0 +
+        // dH) - m0 x H0 = (m0 + d) x dH + d x H0, and the same for m x (m x H)
+        const float m1 = (float)m.b, m2 = (float)m.c, H1 = (float)(h.b * ig), H2 = (float)(h.c * ig),
+                    P1 = (float)(cross_b(m, h) * ig), P2 = (float)(cross_c2(m, h) * ig);
+        auto cross32 = [&](float a1, float a2, float b) {
+          return a1 * dpp_f<QP_ROT2>(b) - a2 * dpp_f<QP_ROT1>(b);
+        };
+        auto delta = [&](float d, float dd) __attribute__((always_inline)) -> float {
+          const float d1 = dpp_f<QP_ROT1>(d), d2 = dpp_f<QP_ROT2>(d), s1 = m1 + d1, s2 = m2 + d2;
+          float dH = fmaf(-p_nms, d, dd);
+          if (CMTJ_HAS(F_ANIS)) dH = fmaf(p_ak, fmaf(p_an2, d2, fmaf(p_an1, d1, p_an * d)), dH);
+          const float dP = cross32(s1, s2, dH) + fmaf(d1, H2, -d2 * H1);
+          const float dQ = cross32(s1, s2, dP) + fmaf(d1, P2, -d2 * P1);
+          return fmaf(dQ, p_al, dP) * p_g;
+        };
+        const float d2 = (float)(k1 * 0.5);
+        float dk = delta(d2, dmid), acc = dk * 2.f;
+        dk = delta(d2 + dk * 0.5f, dmid);
+        acc = acc + dk * 2.f;
+        acc = acc + delta((float)k1 + dk, dend);
+        mn = m.a + k1 + (double)(acc * (float)(1.0 / 6.0));
+      } else {
+        const StageConst KF{(float)K.A0.a, (float)K.A0.b, (float)K.A0.c, (float)K.alpha};
+        mn = m.a + fma((double)stage_increments<DG>(KF, (float)k1, m, h, gb, gc, dmid, dend), 1.0 / 6.0, k1);
+      }
     }
     // ---- CVector::normalize (core/cvector.hpp:185-192).  Binary64: |m|^2 - 1
     // as a butterfly over the quad, (x^2 + y^2) + (z^2 - 1) in all its lanes,
@@ -1485,7 +1536,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
       if (!nb_step) neighbours(nb, m.a);
       const double v = lane_value();
       if (wlog) log_put(f32log, pk, v);
-      if (LOGF == 0 && strip) {
+      if (LOGF != 1 && strip) {
         // stripMagnetoResistance (:1835-1857), parallel sum of the layers
         double rx = 0.0, ry = 0.0;
         if (lact && c == 0) {

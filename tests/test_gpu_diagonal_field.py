@@ -61,5 +61,5 @@ def test_axes(nl, stt, lanes, precision):
     # alone (or among axis-aligned ones) and beside tilted axes
     b, m = out[True]
     for q in (0, 1, 2, 5):
-        a = b.subset(np.array([q])).set_lanes(lanes)
+        a = b.subset(np.array([q]), log_dtype="f64").set_lanes(lanes)
         np.testing.assert_array_equal(a.run().final_m.cpu().numpy()[0, :nl], m[q, :nl])
