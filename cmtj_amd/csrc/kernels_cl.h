@@ -841,18 +841,18 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   [[maybe_unused]] double gw[GP][GS];
   [[maybe_unused]] double g_s = 0.0;
   [[maybe_unused]] int g_buf = 0;
-  [[maybe_unused]] bool g_lane = false, g_sink = false;  // the lane holds a component of the top layer; its m
+  [[maybe_unused]] bool g_lane = false, g_sink = false;  // the lane holds a component of a coupled top layer; its m
   __shared__ GroupClLds<(GW > 0 ? GW : 1), (GW > 0 ? 64 / LPI : 1)> glds;
   if constexpr (GW > 0) {
-    g_lane = live && ly == g_top;
+    // an uncoupled group takes no field whatever its positions: nothing is
+    // checked about them, and two elements may share one
+    g_lane = live && ly == g_top && gp->interaction != CMTJ_INTERACTION_NULL;
     g_sink = c < 3 && ly == g_top;
     const int o = (int)(threadIdx.x & 7u);
     if (g_lane) {
       const cmtj_layer& Ly = g.layers[J->layer_offset + g_top];
       const double V = Ly.thickness * Ly.cell_surface;
-      g_s = (gp->interaction == CMTJ_INTERACTION_KANAO)    ? (Ly.Ms / g.c.mu0) * V
-            : (gp->interaction == CMTJ_INTERACTION_NOMURA) ? Ly.Ms * V / g.c.mu0 / (4 * M_PI)
-                                                           : 0.0;  // nullDipoleInteraction
+      g_s = (gp->interaction == CMTJ_INTERACTION_KANAO) ? (Ly.Ms / g.c.mu0) * V : Ly.Ms * V / g.c.mu0 / (4 * M_PI);
     }
 #pragma unroll
     for (int p = 0; p < GP; ++p) {
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
         const int ei = on ? e : 0, ji = on ? j : 0;
         const double dx = gp->pos[ei][0] - gp->pos[ji][0], dy = gp->pos[ei][1] - gp->pos[ji][1],
                      dz = gp->pos[ei][2] - gp->pos[ji][2];
-        // the host has checked |r| against the reference's limits
+        // the host has checked a coupled group's |r| against the reference's limits
         const double il = on ? 1.0 / sqrt(dx * dx + dy * dy + dz * dz) : 0.0, il2 = il * il;
         const double f = sqrt(3.0 * (il2 * il)) * il;
         gu[p][s] = {dx * f, dy * f, dz * f};
