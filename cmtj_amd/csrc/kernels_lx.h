@@ -18,9 +18,9 @@
 // 0.81 -> 0.62 ms, 196,608 points 2.10 -> 1.94 ms for 2,000 steps at most),
 // and with a diagonal field matrix 111 (65,536 points, 2,000 to 20,000 steps,
 // 7.4 -> 6.7 ms).  Against the general form (kernels_ll.h): RK4 372 -> 111 VALU
-// instructions (20.7 -> 6.7 ms with the waves paired), Euler-Heun 425 -> 254 (131,072 instances x 10,000 steps 24.9 -> 13.3 ms; a
+// instructions (20.7 -> 6.7 ms with the waves paired), Euler-Heun 425 -> 257 (131,072 instances x 10,000 steps 24.9 -> 14.0 ms; a
 // single wave of instances 1.14 -> 0.5 us per step; in binary64 with the same
-// normals also 254, and more registers).
+// normals 1.68 us per step of the 131,072 against 1.45: 222 registers).
 // WPE: waves per SIMD the register allocation must leave room for.
 #pragma once
 
@@ -334,7 +334,11 @@ k_junction_lx(GroupArgs g) {
       };
       const V3<R> k0 = kick(mr);
       const V3<R> k1 = kick(mr + k0);
-      mn = m + cvt<double>(axpy(R(0.5), k0 + k1, f));
+      // drift and kick are added to m each in binary64: a kick far below the
+      // drift would be lost in a binary32 sum (three conversions fewer, 13.4
+      // against 14.0 ms)
+      const V3<double> md = m + cvt<double>(f);
+      mn = axpy(0.5, cvt<double>(k0 + k1), md);
     }
     // ---- CVector::normalize (core/cvector.hpp:185-192): (1 + e)^(-1/2) by its
     // series up to |e| = kUnitRange, exactly beyond
