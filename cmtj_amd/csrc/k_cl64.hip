@@ -6,6 +6,12 @@ namespace cmtj {
 static const KEntry kC64[] = {
     CMTJ_KC64(2, FM_PIMM, 1),  CMTJ_KC64(2, FM_PIMM, -1), CMTJ_KC64(4, FM_PIMM, -1), CMTJ_KC64(1, FM_RH, 0),
     CMTJ_KC64(1, FM_VSD, 1),   CMTJ_KC64(1, FM_LEAN, -1), CMTJ_KC64(2, FM_LEAN, -1), CMTJ_KC64(4, FM_LEAN, -1),
+    // constant and sine fields alone (without this set FM_FIELD, whose kind of
+    // drive is compiled in too, ranks before FM_LEAN; us per step: 101 bilayers
+    // in a constant field 0.57 with FM_FIELD, 0.30 with FM_LEAN, 0.32 here; 1023
+    // in a sine field 0.77, 0.66, 0.42; 512 one-layer devices under two sines
+    // 0.70, 0.88, 0.39)
+    CMTJ_KC64(1, FM_LEAN_SINE, -1), CMTJ_KC64(2, FM_LEAN_SINE, -1), CMTJ_KC64(4, FM_LEAN_SINE, -1),
     // spin torques, scalar drives: the STO set and the lean set with both
     CMTJ_KC64(2, FM_STO, -1),
     // RK4 also reads callback drivers sampled at its three stage times

@@ -33,6 +33,7 @@ constexpr uint32_t FM_SOTT = F_ANIS | F_IEC | F_DYN | F_DYNH | F_SOT | F_THERMAL
 constexpr uint32_t FM_STTC = F_ANIS | F_ANIS2 | F_IEC | F_IEC2 | F_DEMAG_OFF | F_IDMI | F_DIPOLE | F_DYNH | F_DYN |
                              F_STT | F_SOT | F_SOT2;
 constexpr uint32_t FM_FIELD = (FM_STTC & ~(F_STT | F_SOT | F_SOT2)) | F_KSINE;
+constexpr uint32_t FM_LEAN_SINE = FM_LEAN | F_KSINE;
 // coupled runs (stacks, groups): the usual member's features
 constexpr uint32_t FM_STATIC = F_ANIS | F_IEC;  // the lean set under constant drives
 constexpr uint32_t FM_CPL = F_ANIS | F_IEC | F_DYN | F_DYNH | F_STT | F_SOT | F_THERMAL;
