@@ -224,6 +224,7 @@ EXPORTS = (
     "cmtj_abi",
     "cmtj_last_error",
     "cmtj_last_kernels",
+    "cmtj_last_side_set",
     "cmtj_constants_get",
     "cmtj_constants_set",
     "cmtj_constants_reset",
@@ -336,6 +337,12 @@ def last_error() -> str:
 def last_kernels() -> list[str]:
     """Kernels the calling thread's last engine run launched."""
     return [k for k in (lib().cmtj_last_kernels() or b"").decode().split(";") if k]
+
+
+def last_side_set() -> int:
+    """Stream set of the calling thread's last plan execute, -1: its groups
+    ran on the caller's stream alone."""
+    return int(lib().cmtj_last_side_set())
 
 
 def ptr(a: np.ndarray | None) -> int | None:

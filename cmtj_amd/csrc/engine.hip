@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -23,6 +24,7 @@ using namespace cmtj;
 
 static thread_local std::string g_err;
 static thread_local std::string g_last_kernels;  // kernels of the calling thread's last launch
+static thread_local int g_last_set = -1;         // stream set of its last cmtj_plan_execute
 
 static int fail(int code, const std::string& msg) {
   g_err = msg;
@@ -598,6 +600,21 @@ namespace {
 constexpr int kSideStreams = 3;  // with the caller's stream the four hardware queues of a process
 constexpr int kSideSets = 4;     // per device
 
+// A caller's stream: its handle and, for the per-thread stream, whose handle
+// every thread's own one shares, the thread's number.  (A handle may also come
+// back after hipStreamDestroy, which waits for the stream's work: 100 ms of it
+// took the call 100 ms, three times of three.)
+struct UserStream {
+  hipStream_t s = nullptr;
+  uint64_t thread = 0;
+  bool operator==(const UserStream& o) const { return s == o.s && thread == o.thread; }
+};
+UserStream user_stream(hipStream_t s) {
+  static std::atomic<uint64_t> count{0};
+  static thread_local const uint64_t number = ++count;  // (a thread's id may come back)
+  return {s, s == hipStreamPerThread ? number : 0};
+}
+
 // Streams and events of one fork.  A set is taken for the enqueueing of one
 // execute and reused for the same caller's stream, whose order its joins are
 // part of already, or when the work last put on it is done (otherwise one
@@ -608,7 +625,8 @@ struct SideSet {
   hipEvent_t fork = nullptr, join[kSideStreams] = {};
   bool used[kSideStreams] = {};  // the joins of the last execute
   bool taken = false;
-  hipStream_t user = nullptr;  // the caller's stream of the last execute
+  UserStream user;  // the caller's stream of the last execute
+  int index = 0;    // in the device's pool
 };
 struct SidePool {
   std::mutex mu;
@@ -643,6 +661,7 @@ bool make_set(SideSet& t) {
 }
 
 SideSet* take_set(hipStream_t s) {
+  const UserStream user = user_stream(s);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   const RelaxedCapture relaxed;
@@ -650,7 +669,7 @@ SideSet* take_set(hipStream_t s) {
   std::lock_guard<std::mutex> lk(pool.mu);
   auto& v = pool.sets[dev];
   for (auto& t : v)
-    if (!t->taken && t->user == s) {
+    if (!t->taken && t->user == user) {
       t->taken = true;
       return t.get();
     }
@@ -663,7 +682,7 @@ SideSet* take_set(hipStream_t s) {
         idle = false;
       }
     if (idle) {
-      t->user = s;
+      t->user = user;
       t->taken = true;
       return t.get();
     }
@@ -671,8 +690,9 @@ SideSet* take_set(hipStream_t s) {
   if (v.size() >= (size_t)kSideSets) return nullptr;
   std::unique_ptr<SideSet> t(new SideSet);
   if (!make_set(*t)) return nullptr;
-  t->user = s;
+  t->user = user;
   t->taken = true;
+  t->index = (int)v.size();
   v.push_back(std::move(t));
   return v.back().get();
 }
@@ -716,6 +736,7 @@ bool spread_groups(const cmtj_plan& P, std::vector<int>& lane_of) {
 int launch_spread(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_status, hipStream_t s) {
   std::vector<int> lane_of;
   std::unique_ptr<SideSet, GiveBack> t;
+  g_last_set = -1;
   if (spread_groups(*P, lane_of)) {
     // a capturing stream keeps the launches on itself: forked streams would
     // stay part of the capture until it ends
@@ -730,6 +751,7 @@ int launch_spread(cmtj_plan* P, void* d_log, double* d_mag, cmtj_status* d_statu
     }
   }
   if (!t) return launch_plan(P, d_log, d_mag, d_status, s);
+  g_last_set = t->index;
   void* streams[1 + kSideStreams] = {(void*)s};
   bool used[kSideStreams] = {};
   for (int l : lane_of)
@@ -893,6 +915,7 @@ int cmtj_abi(cmtj_abi_info* out) {
 
 const char* cmtj_last_error(void) { return g_err.c_str(); }
 const char* cmtj_last_kernels(void) { return g_last_kernels.c_str(); }
+int cmtj_last_side_set(void) { return g_last_set; }
 
 int cmtj_constants_get(cmtj_constants* out) {
   if (!out) return fail(CMTJ_ERR_INVALID, "null pointer");

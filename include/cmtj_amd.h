@@ -277,6 +277,13 @@ const char* cmtj_last_error(void);
  * chose. */
 const char* cmtj_last_kernels(void);
 
+/* Stream set on which the calling thread's last cmtj_plan_execute ran its
+ * structure groups side by side (0, 1, ... per device), -1 where it ran them
+ * on the caller's stream alone: a single group, groups that fill the chip or
+ * are too short, a capturing stream, or every set in use.  No counterpart in
+ * the reference. */
+int cmtj_last_side_set(void);
+
 /* Process-wide constants store behind the Python PhysicalConstants class.
  * Replaces the static members and setters/getters of
  * core/constants.hpp:6-53 (bound at python/cmtj.cpp:496-511). */
