@@ -52,7 +52,7 @@ struct Mat3 {
 // engine.hip).
 template <class R, int L, int SOLVER, uint32_t FM, int WPE = 1, int ND = -1>
 __global__ __launch_bounds__(SOLVER == CMTJ_RK4 ? 256 * WPE : 64) __attribute__((amdgpu_waves_per_eu(WPE))) void
-k_junction_lx(GroupArgs g) {
+k_junction_ll_exact(GroupArgs g) {
   constexpr bool RK4 = SOLVER == CMTJ_RK4;
   static_assert(L == 2 || L == 4, "L lanes per instance must divide a 16-lane DPP row");
   static_assert(FM & F_EXACT, "exact feature sets");

@@ -78,8 +78,8 @@ KTable kernels_group_cl();  // Kanao / Nomura groups on one lane per component
 
 // the large batches' exact sets (kernels_lx.h), the register allocation capped for WPE waves per SIMD
 #define CMTJ_KLX(R, PREC, L, S, FM, WPE, ND)                                                \
-  {PREC, L, L, S, FM, false, (const void*)&cmtj::k_junction_lx<R, L, S, FM, WPE, ND>,       \
-   "k_junction_ll<" #R "," #L "," #S "," #FM "," #ND ",waves " #WPE ">", (ND) + 1, 0,       \
+  {PREC, L, L, S, FM, false, (const void*)&cmtj::k_junction_ll_exact<R, L, S, FM, WPE, ND>,       \
+   "k_junction_ll_exact<" #R "," #L "," #S "," #FM "," #ND ",waves " #WPE ">", (ND) + 1, 0,       \
    (S) == CMTJ_RK4 ? 4 * (WPE) : 0}
 
 #define CMTJ_KC(L, FM, ND)                                                                     \
