@@ -110,7 +110,15 @@ _LANES = {"auto": 0, "one": 1, "per_layer": 2, "per_component": 3, "queue": 4}
 
 
 class JunctionBatch:
-    """A packed batch of junction instances (see module docstring)."""
+    """A packed batch of junction instances (see module docstring).
+
+    log_dtype ("f32" by default for FP32 batches, "f64" for FP64 ones) is the
+    type of the log's entries.  In FP32 batches of anisotropy, bilinear
+    coupling and field drives other than steps it also chooses between two
+    forms of the binary32 increments, so the final m of a run with "f32"
+    entries differs from that with "f64" ones by some 1e-8 (a sine field,
+    5,000 steps: 4.8e-9 and 2.0e-8 from the FP64 run, 0.26 and 1.32 us per
+    step).  ``subset`` takes the default unless told otherwise."""
 
     def __init__(self, js, layers, tables, metas, meta_index, precision="fp32", log="full", log_dtype=None):
         self.js = js
@@ -324,7 +332,8 @@ class JunctionBatch:
         one GPU lane), "per_layer" (one lane per layer), "per_component" (one
         lane per vector component of each layer: binary32 RK4 groups of the
         lean feature set; binary64 groups of every feature but energy
-        channels), "auto" (per component where such a kernel covers
+        channels; FP32 Euler-Heun and Heun groups run per layer when asked for
+        components, and per component by "auto" only), "auto" (per component where such a kernel covers
         the group and the batch leaves SIMDs idle, else per layer for
         multilayer instances) or "queue" (single-layer Dormand-Prince groups
         on a persistent grid whose lanes take instances from a device work
@@ -371,11 +380,13 @@ class JunctionBatch:
 
     @property
     def fp64_groups(self) -> int:
-        """Structure groups of an FP32 batch that run binary64 kernels (spin
-        torques or scalar drives on one lane per component, where no
-        binary32 kernel covers them): their arithmetic is the drop-in's.
-        (The layer-lane RK4 set of anisotropy, coupling and field steps has
-        binary64 steps in both modes and is not counted.)"""
+        """Structure groups of an FP32 batch that run a kernel of the FP64
+        mode (spin torques or scalar drives on one lane per component, where
+        the FP32 mode has no kernel): their arithmetic is the drop-in's.
+        Kernels of the FP32 mode are not counted, also where their steps are
+        binary64: the layer-lane RK4 set of anisotropy, coupling and field
+        steps, and Euler-Heun and Heun on one lane per component (with
+        binary32 normals)."""
         return int(self.plan().info.fp64_groups)
 
     def capture(self, device="cuda") -> "JunctionBatch":

@@ -578,11 +578,14 @@ __global__ __launch_bounds__(64 * (GW > 0 ? GW : 1)) void k_junction_cl(GroupArg
   constexpr bool DGSET = SOLVER == CMTJ_RK4 && !(FM & (F_DEMAG_OFF | F_IEC2));
   const bool diag = DGSET && __ballot(K.A0.b != 0.0 || K.A0.c != 0.0 || K.A1.a != 0.0 || K.A1.c != 0.0 ||
                                       K.A2.a != 0.0 || K.A2.b != 0.0) == 0ull;
-  // Binary32 sets that take waveforms keep the form of their increments and
-  // their single-precision waveforms where entries are binary64, in which
-  // another order of the binary32 operations shows (3e-9 of m after 5,000
-  // steps); with binary32 entries they take the shorter ones (LOGF 2; a sine
-  // field's step 1.3 -> 0.3 us).
+  // Binary32 sets that take waveforms run in two forms, by the log's entries.
+  // With binary32 entries (LOGF 2): carried binary64 phases and the increments
+  // of stage_increments.  With binary64 entries: single-precision waveforms and
+  // increments about the anchor in the lane's own order, the slower form and
+  // the one further off (256 one-layer instances under a sine field x 5,000
+  // steps: 1.32 against 0.26 us per step, 2.0e-8 against 4.8e-9 of m from the
+  // binary64 run), kept so that binary64 entries keep their values to 1e-9: the
+  // other form moves them by 3e-8.
   constexpr bool PLAIN32 = !F64 && LOGF != 2 && !(FM & F_KSTEP);
   [[maybe_unused]] float p_an = 0, p_an1 = 0, p_an2 = 0, p_nms = 0, p_ak = 0, p_al = 0, p_g = 0;
   [[maybe_unused]] double ig = 0.0;

@@ -465,9 +465,14 @@ typedef struct cmtj_plan_info {
   int32_t max_layers;       /* largest layer count in the batch */
   int32_t n_kernels;        /* kernel launches per execute */
   int32_t lanes_per_instance;
-  int32_t fp64_groups;      /* CMTJ_FP32 plans: groups that run a binary64 kernel
-                               (spin torques or scalar drives on one lane per
-                               component, where no binary32 kernel covers them) */
+  int32_t fp64_groups;      /* CMTJ_FP32 plans: groups that run a kernel of the
+                               CMTJ_FP64 mode (spin torques or scalar drives on
+                               one lane per component, where the CMTJ_FP32 mode
+                               has no kernel).  Kernels of the CMTJ_FP32 mode
+                               are not counted, also where their steps are
+                               binary64: layer-lane RK4 of anisotropy, coupling
+                               and field steps, component-lane Euler-Heun and
+                               Heun (with binary32 normals) */
   char kernel_name[128];
 } cmtj_plan_info;
 
@@ -482,7 +487,9 @@ typedef struct cmtj_plan_info {
  * lane), CMTJ_LANES_PER_LAYER (one lane per layer, for multilayer
  * instances), CMTJ_LANES_PER_COMPONENT (four lanes per layer, one per vector
  * component: binary32 RK4 groups of the lean feature set; binary64 groups of
- * every feature but energy channels, with RK4, Heun or Euler-Heun) or CMTJ_LANES_AUTO
+ * every feature but energy channels, with RK4, Heun or Euler-Heun; CMTJ_FP32
+ * Heun and Euler-Heun groups run per layer when asked for components and per
+ * component by CMTJ_LANES_AUTO only) or CMTJ_LANES_AUTO
  * (one lane per component where such a kernel covers the group and its waves
  * fit one per SIMD, else one lane per layer for multilayer instances).
  * Returns NULL on error (see cmtj_last_error). */
