@@ -647,7 +647,7 @@ def main() -> int:
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported "
-              "(instances shard across GPUs with no exchange; see DESIGN.md)", file=sys.stderr)
+              "(instances shard across GPUs with no exchange)", file=sys.stderr)
         return 2
 
     import numpy as np

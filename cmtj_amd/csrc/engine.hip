@@ -129,7 +129,7 @@ static const KEntry* pick_kernel(int prec, int nl, int solver, uint32_t flags, u
   // sweep is its longest instance's step count times the latency of one
   // wave step.  One lane per component issues about half the instructions
   // per wave step of one lane per layer, and at four times the lanes spreads
-  // over more SIMDs (PIMM set: 94 against 111 VALU a step): it wins while its waves still fit one per
+  // over more SIMDs (PIMM set: 100 against 114 VALU a step): it wins while its waves still fit one per
   // SIMD, and costs several times the instructions per junction-step beyond that
   // (FP32 Euler-Heun, us per step: 8,192 two-layer switching devices 0.41
   // against 0.53, 16,384 0.65 against 0.55; 4,096 four-layer chains 0.90
@@ -139,7 +139,7 @@ static const KEntry* pick_kernel(int prec, int nl, int solver, uint32_t flags, u
   // smaller than one lane per instance's, so more waves fit per SIMD, and the
   // exact sets of large batches have their leanest kernels there (65,536-point
   // PIMM sweep 1.1e11 junction-steps/s against 2.4e10 with one lane per
-  // instance, 131,072-instance CIMS ensemble 9.8e10 against 6.3e10).
+  // instance, 131,072-instance CIMS ensemble 9.4e10 against 6.3e10).
   if (best[1] && (nl >= 2 || !best[0])) return best[1];
   if (best[0]) return best[0];
   return best[1] ? best[1] : best[2];
@@ -1271,8 +1271,8 @@ int cmtj_run_groups(const cmtj_group* groups, size_t n_groups, const cmtj_juncti
                 "the junctions of a group must share one structure (layers, modes, driver kinds)");
   // The smallest group kernel that covers the structure.  Point-dipole
   // coupling: one lane per component, in as few waves as hold the elements
-  // (faster at every size: one group of 64 elements 3.6 -> 0.9 us per step,
-  // of 9 4.0 -> 0.9 us, 512 groups of 64 202 -> 186 us).
+  // (faster at every size: one group of 64 elements 3.3 -> 0.68 us per step,
+  // 1024 of them 6.1 -> 3.0 us).
   // Otherwise (tensor coupling, whose pair terms do not fit in registers,
   // more features, Euler-Heun) one lane per element: four waves per group
   // while the groups leave SIMDs idle (the sum over the sources then takes a

@@ -11,10 +11,11 @@
 // cross product are formed in the lane; what crosses lanes is each stage's m
 // and, once per step, the neighbour layers' (start-of-step values,
 // core/junction.hpp:1682-1707) by a row shift of 4 lanes.  A step of one wave
-// issues about a third of the instructions of the one-layer-per-lane kernel,
-// and a batch occupies four times as many waves: on a batch too small to fill
-// the chip both shorten the sweep, whose time is the step count of the longest
-// instance times the latency of one wave step.
+// issues fewer instructions than one layer per lane (PIMM set 100 against 114
+// VALU, the binary64 step among the latter), and a batch occupies four times
+// as many waves: on a batch too small to fill the chip both shorten the sweep,
+// whose time is the step count of the longest instance times the latency of one
+// wave step.
 //
 // Integrators: the anchored binary32 RK4 of the other FP32 kernels (rk4_step,
 // core/junction.hpp:1017-1041): k1 and the state in binary64, stages 2-4 as

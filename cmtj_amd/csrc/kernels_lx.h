@@ -18,7 +18,8 @@
 // 0.81 -> 0.62 ms, 196,608 points 2.10 -> 1.94 ms for 2,000 steps at most),
 // and with a diagonal field matrix 111 (65,536 points, 2,000 to 20,000 steps,
 // 7.4 -> 6.7 ms).  Against the general form (kernels_ll.h): RK4 372 -> 111 VALU
-// instructions (20.7 -> 6.7 ms with the waves paired), Euler-Heun 425 -> 257 (131,072 instances x 10,000 steps 24.9 -> 14.0 ms; a
+// instructions (20.7 -> 6.7 ms with the waves paired), Euler-Heun 425 -> 257 in
+// the loop's code, 244 counted (131,072 instances x 10,000 steps 24.9 -> 14.0 ms; a
 // single wave of instances 1.14 -> 0.5 us per step; in binary64 with the same
 // normals 1.68 us per step of the 131,072 against 1.45: 222 registers).
 // WPE: waves per SIMD the register allocation must leave room for.
